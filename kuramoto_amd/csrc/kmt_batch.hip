@@ -90,7 +90,8 @@ __global__ __launch_bounds__(kBlock) void bsincos_kernel(const float *y, const B
   const long n = (long)blockIdx.x * kBlock + threadIdx.x;
   if (n >= inst[b].n) return;
   const float v = y[(size_t)b * ldn + n];
-  const float c = rcos<float>(v), s = rsin<float>(v);
+  float c, s;
+  rsincos<float>(v, c, s);
   cs[((size_t)b * 2) * ldn + n] = c;
   cs[((size_t)b * 2 + 1) * ldn + n] = s;
   if (write_vt) put_vt<T>(vt, inst[b].vrow, n, c, s);
@@ -534,7 +535,8 @@ __global__ __launch_bounds__(kBlock) void bepilogue_kernel(const BVecs a) {
       }
       const float yt = rfma<float>(acc, h, a.y[vb + n]);
       if constexpr (s + 1 == 7) a.ynew[vb + n] = yt;
-      const float c = rcos<float>(yt), si = rsin<float>(yt);
+      float c, si;
+      rsincos<float>(yt, c, si);
       a.cs_out[2 * vb + n] = c;
       a.cs_out[2 * vb + a.ldn + n] = si;
       if (a.write_vt) put_vt<T>(a.vt, in->vrow, n, c, si);
@@ -736,7 +738,8 @@ __global__ __launch_bounds__(kBlock) void bemit_kernel(const BEmit a) {
   const float h = in->h;
   auto stage2 = [&](float yv, float k1) {
     const float yt = rfma<float>(k1 * (float)tab::A[0][0], h, yv);
-    const float c = rcos<float>(yt), s = rsin<float>(yt);
+    float c, s;
+    rsincos<float>(yt, c, s);
     a.cs_out[2 * vb + n] = c;
     a.cs_out[2 * vb + a.ldn + n] = s;
     if (a.write_vt) put_vt<T>(a.vt, in->vrow, n, c, s);
@@ -764,8 +767,10 @@ __global__ __launch_bounds__(kBlock) void bemit_kernel(const BEmit a) {
       double cx = 0, sx = 0;
       if (valid) {
         const float val = dense_value<float>(Q, yl, hh, x);
-        cx = (double)rcos<float>(val);
-        sx = (double)rsin<float>(val);
+        float c, s;
+        rsincos<float>(val, c, s);
+        cx = (double)c;
+        sx = (double)s;
       }
       const double bc = block_sum(cx, sh), bs = block_sum(sx, sh);
       if (threadIdx.x == 0) {

@@ -137,11 +137,14 @@ template <class R, int VEC> __device__ __forceinline__ void load_reals(const R *
 // the same way).  With Cauchy frequencies the fast oscillators' phases
 // reach 1e4, where one float ulp is 1e-3 rad, and a last-bit difference of
 // a cos or sin moves the whole population by ~1e-4 within t = 1.
-template <class R> __device__ __forceinline__ R rcos(R x) {
-  if constexpr (sizeof(R) == 4) return (float)cos((double)x); else return cos(x);
-}
-template <class R> __device__ __forceinline__ R rsin(R x) {
-  if constexpr (sizeof(R) == 4) return (float)sin((double)x); else return sin(x);
+// Both come from one sincos: the same bits as cos() and sin() (compared over
+// 2^31 arguments of every range), which each reduce the argument again (214
+// against 111 double operations).
+template <class R> __device__ __forceinline__ void rsincos(R x, R &c, R &s) {
+  double ds, dc;
+  sincos((double)x, &ds, &dc);
+  c = (R)dc;
+  s = (R)ds;
 }
 template <class R> __device__ __forceinline__ R rabs(R x) {
   if constexpr (sizeof(R) == 4) return fabsf(x); else return fabs(x);
@@ -232,8 +235,10 @@ __device__ __forceinline__ double row_epilogue(const Vecs<R> &a, long i, R C, R 
       }
       const R yt = rfma<R>(acc, h, a.y[i]);
       if constexpr (s + 1 == 7) a.ynew[i] = yt;
-      a.cs_out[i] = rcos<R>(yt);
-      a.cs_out[a.ldv + i] = rsin<R>(yt);
+      R c, sn1;
+      rsincos<R>(yt, c, sn1);
+      a.cs_out[i] = c;
+      a.cs_out[a.ldv + i] = sn1;
       return 0.0;
     } else {
       // embedded error, dp45.cu:79-84
@@ -902,8 +907,10 @@ template <class R> __device__ __forceinline__ R dense_value(const R Q[4], R yl, 
 
 template <class R> __device__ __forceinline__ void stage2_vector(const EmitArgs<R> &a, long i, R y, R k1, R h) {
   const R yt = rfma<R>(k1 * (R)tab::A[0][0], h, y);
-  a.cs_out[i] = rcos<R>(yt);
-  a.cs_out[a.ldv + i] = rsin<R>(yt);
+  R c, s;
+  rsincos<R>(yt, c, s);
+  a.cs_out[i] = c;
+  a.cs_out[a.ldv + i] = s;
 }
 
 template <class R>
@@ -941,8 +948,10 @@ __global__ __launch_bounds__(kBlock) void emit_commit_kernel(const EmitArgs<R> a
       if (valid) {
         const R val = dense_value<R>(Q, yl, hh, x);
         if (a.ring) a.ring[(size_t)slot * a.ldv + i] = val;
-        cx = (double)rcos<R>(val);
-        sx = (double)rsin<R>(val);
+        R c, s;
+        rsincos<R>(val, c, s);
+        cx = (double)c;
+        sx = (double)s;
       }
       const double bc = block_sum(cx, sh);
       const double bs = block_sum(sx, sh);
@@ -1010,8 +1019,10 @@ template <class R>
 __global__ __launch_bounds__(kBlock) void sincos_kernel(const R *y, long N, long ldv, R *cs) {
   const long i = (long)blockIdx.x * kBlock + threadIdx.x;
   if (i < N) {
-    cs[i] = rcos<R>(y[i]);
-    cs[ldv + i] = rsin<R>(y[i]);
+    R c, s;
+    rsincos<R>(y[i], c, s);
+    cs[i] = c;
+    cs[ldv + i] = s;
   }
 }
 
@@ -1021,9 +1032,10 @@ template <class R>
 __global__ __launch_bounds__(kBlock) void sincos_pad_kernel(const R *y, long N, long ldv, R *cs) {
   const long i = (long)blockIdx.x * kBlock + threadIdx.x;
   if (i < ldv) {
-    const bool in = i < N;
-    cs[i] = in ? rcos<R>(y[i]) : (R)0;
-    cs[ldv + i] = in ? rsin<R>(y[i]) : (R)0;
+    R c = 0, s = 0;
+    if (i < N) rsincos<R>(y[i], c, s);
+    cs[i] = c;
+    cs[ldv + i] = s;
   }
 }
 
@@ -1032,7 +1044,12 @@ __global__ __launch_bounds__(kBlock) void order_partial_kernel(const R *y, long 
   __shared__ double sh[kBlock];
   const long i = (long)blockIdx.x * kBlock + threadIdx.x;
   double c = 0, s = 0;
-  if (i < N) { c = (double)rcos<R>(y[i]); s = (double)rsin<R>(y[i]); }
+  if (i < N) {
+    R cy, sy;
+    rsincos<R>(y[i], cy, sy);
+    c = (double)cy;
+    s = (double)sy;
+  }
   const double bc = block_sum(c, sh);
   const double bs = block_sum(s, sh);
   if (threadIdx.x == 0) { part[2 * blockIdx.x] = bc; part[2 * blockIdx.x + 1] = bs; }
