@@ -730,7 +730,7 @@ __global__ __launch_bounds__(kBlock) void bemit_kernel(const BEmit a) {
   const int b = blockIdx.y;
   const BInst *in = a.inst + b;
   if (!in->active) return;
-  __shared__ double sh[kBlock];
+  __shared__ double sh[kEmitRows][2][kBlock];
   const long n = (long)blockIdx.x * kBlock + threadIdx.x;
   const bool valid = n < in->n;
   const size_t vb = (size_t)b * a.ldn;
@@ -761,24 +761,12 @@ __global__ __launch_bounds__(kBlock) void bemit_kernel(const BEmit a) {
       dense_coeffs<float>(kv, Q);
       yl = a.y[vb + n];
     }
-    for (int q = 0; q < n_emit; ++q) {
-      const int slot = in->ring_count + q;
-      const float x = (a.t_eval[in->pend_lo + q] - tl) / hh;
-      double cx = 0, sx = 0;
-      if (valid) {
-        const float val = dense_value<float>(Q, yl, hh, x);
-        float c, s;
-        rsincos<float>(val, c, s);
-        cx = (double)c;
-        sx = (double)s;
-      }
-      const double bc = block_sum(cx, sh), bs = block_sum(sx, sh);
-      if (threadIdx.x == 0) {
-        const size_t o = (((size_t)b * a.ring_cap + slot) * a.nblk + blockIdx.x) * 2;
-        a.ord_part[o] = bc;
-        a.ord_part[o + 1] = bs;
-      }
-    }
+    const int slot0 = in->ring_count, lo = in->pend_lo;
+    emit_rows<float>(
+        n_emit, valid, Q, yl, tl, hh, sh, [&](int q) { return a.t_eval[lo + q]; }, [](int, float) {},
+        [&](int q) {
+          return reinterpret_cast<double2 *>(a.ord_part) + ((size_t)b * a.ring_cap + slot0 + q) * a.nblk + blockIdx.x;
+        });
   }
   if (n_emit == pend && valid) {
     const float yo = a.y[vb + n], yn = a.ynew[vb + n], k7 = a.kbuf[6 * kst + vb + n];
@@ -796,29 +784,16 @@ __global__ __launch_bounds__(kBlock) void bfinalize_kernel(BInst *inst, const do
   const int b = blockIdx.x;
   BInst *in = inst + b;
   if (!in->active || !in->commit_pending) return;
-  __shared__ double sh[kBlock];
   const int pend = in->pend_hi - in->pend_lo;
   const int room = ring_cap - in->ring_count;
   const int n_emit = pend < room ? pend : room;
   const int base = in->ring_count;
-  float r_last = in->r_now, r_before = in->r_prev;
-  for (int q = 0; q < n_emit; ++q) {
-    const int slot = base + q;
-    double sx = 0, sy = 0;
-    for (int x = threadIdx.x; x < nblk; x += kBlock) {
-      const size_t o = (((size_t)b * ring_cap + slot) * nblk + x) * 2;
-      sx += ord_part[o];
-      sy += ord_part[o + 1];
-    }
-    const double X = block_sum(sx, sh), Y = block_sum(sy, sh);
-    const float r = order_value<float>(X, Y, in->n);
-    if (threadIdx.x == 0) r_ring[(size_t)b * ring_cap + slot] = r;
-    r_before = r_last;
-    r_last = r;
-  }
+  float *r = r_ring + (size_t)b * ring_cap + base;
+  order_rows<float>(n_emit, ord_part + ((size_t)b * ring_cap + base) * nblk * 2, nblk, in->n, r);
   __syncthreads();
   if (threadIdx.x == 0) {
     if (n_emit > 0) {
+      const float r_last = r[n_emit - 1], r_before = n_emit > 1 ? r[n_emit - 2] : in->r_now;
       const int last = in->pend_lo + n_emit - 1;
       in->tr_prev = n_emit > 1 ? t_eval[last - 1] : in->tr_now;
       in->tr_now = t_eval[last];

@@ -1059,7 +1059,7 @@ template <class R> struct Engine : EngineBase {
   }
 
   // One attempt: stages 2..7 (cs ping-pong 0->1->0->1->0->1), control,
-  // emit/commit (writes stage-2 vector into cs[0]), finalize.
+  // emit/commit (writes stage-2 vector into cs[0]).
   void launch_attempt(std::vector<std::pair<hipEvent_t, hipEvent_t>> *ev = nullptr) {
     if (factored == KMT_LOWRANK_CONTRACT && lr_fused()) launch_lr_attempt(ev);
     else for (int s = 2; s <= 7; ++s) {
@@ -1073,10 +1073,13 @@ template <class R> struct Engine : EngineBase {
         ev->erase(ev->begin());
       }
     }
-    control_kernel<R><<<1, kBlock, 0, stream>>>(st, err_part, n_parts_stage7(), N, t_eval, times);
+    control_kernel<R><<<1, kBlock, 0, stream>>>(st, err_part, n_parts_stage7(), N, t_eval, times, ord_part, nblk_emit,
+                                                r_ring);
     emit_commit_kernel<R><<<(unsigned)nblk_emit, kBlock, 0, stream>>>(emit_args());
-    finalize_kernel<R><<<1, kBlock, 0, stream>>>(st, ord_part, nblk_emit, N, r_ring);
   }
+  // the order parameters of the last attempt's rows (earlier ones are
+  // computed by the next attempt's control_kernel): before the host looks
+  void launch_finalize() { finalize_kernel<R><<<1, kBlock, 0, stream>>>(st, ord_part, nblk_emit, N, r_ring); }
 
   int build_graphs() {
     drop_graphs();
@@ -1085,6 +1088,7 @@ template <class R> struct Engine : EngineBase {
       hipGraph_t g = nullptr;
       HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
       for (int a = 0; a < n; ++a) launch_attempt();
+      launch_finalize();
       HIP_TRY(hipStreamEndCapture(stream, &g));
       hipGraphExec_t ex = nullptr;
       hipError_t e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
@@ -1186,6 +1190,7 @@ template <class R> struct Engine : EngineBase {
     shadow.ring_cap = ring_cap;
     shadow.times_cap = times_cap;
     shadow.rhs_evals = 1;
+    shadow.job_mode = shadow.active ? JOB_STAGE2 : JOB_NONE;
     KMT_TRY(push_state());
     if (!tuned && !factored && !sym()) default_variant();
     // k1 = f(y) (dp45.cu:151), then the first stage-2 vector
@@ -1359,6 +1364,7 @@ template <class R> struct Engine : EngineBase {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> work = pairs_all;
     HIP_TRY(hipEventRecord(r0, stream));
     for (int a = 0; a < attempts; ++a) launch_attempt(&work);
+    launch_finalize();
     HIP_TRY(hipEventRecord(r1, stream));
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventSynchronize(r1));

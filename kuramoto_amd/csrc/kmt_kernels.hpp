@@ -1,19 +1,22 @@
 // HIP device code of the integrator (gfx950 / CDNA4, wave64).
 //
-// One DP45 attempt is 9 launches on one stream (captured in a hipGraph):
+// One DP45 attempt is 8 launches on one stream (captured in a hipGraph):
 //   stage_kernel<2..7>  A streamed from HBM once per stage for both cos and
 //                       sin; the epilogue writes k_s and the next stage's
 //                       (cos, sin) of y + h*sum a_{s+1,j} k_j (stage 6 also
 //                       keeps the 5th-order solution; stage 7 forms the
 //                       embedded error and a per-workgroup sum of squares)
 //   control_kernel      error norm, accept/reject, step-size update,
-//                       accepted-step log, output times crossed
+//                       accepted-step log, output times crossed, ring and
+//                       output bookkeeping, end-of-run detection; also the
+//                       order parameter of the rows the previous attempt
+//                       emitted
 //   emit_commit_kernel  dense output at the crossed output times + order
 //                       parameter partial sums, then commit (ylast <- y,
 //                       y <- y5, k1 <- k7) and the next attempt's stage-2
 //                       (cos, sin)
-//   finalize_kernel     order parameter of each emitted row, ring and
-//                       output bookkeeping, end-of-run detection
+// and after the last attempt of a graph
+//   finalize_kernel     order parameter of the rows that attempt emitted
 // Reference counterparts: dp45.cu:34-164 (stages, error, controller, FSAL,
 // interpolation) and kuramoto.cu:42-55, :104-126, :164-249 (RHS, order
 // parameter, output grid).
@@ -64,10 +67,19 @@ template <class R> struct State {
   int fixed;
   int last_accept;
   int error;
-  int pad_;
+  // what emit_commit_kernel has to do for the attempt just controlled: rows
+  // t_eval[job_lo .. job_lo + job_n) into ring slots from job_slot, then
+  // job_mode; the rows' order parameters follow in the next control_kernel
+  // (or finalize_kernel), which then clears fin_n
+  int job_mode, job_lo, job_n, job_slot;
+  int fin_n;
   long long accepted, rejected, attempts, rhs_evals;
   double norm;
 };
+constexpr int JOB_NONE = 0;    // nothing (run finished)
+constexpr int JOB_STAGE2 = 1;  // rejected step or start of a run: stage-2 vector from (y, k1)
+constexpr int JOB_EMIT = 2;    // outputs only (the ring is full before the last one)
+constexpr int JOB_COMMIT = 3;  // outputs, commit, stage-2 vector
 
 // Storage tags for the adjacency.
 struct bf16_t { uint16_t bits; };
@@ -162,16 +174,25 @@ template <class T> __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
-// Deterministic block sum of one double per thread (fixed tree order).
+// Deterministic sum of one double per thread of a workgroup, in a fixed tree:
+// x[t] + x[t + 128], then + 64, 32, ... 1.  The first two levels are read
+// from LDS by one wave, the others are lane exchanges (a barrier per level
+// took about three times as long): block_tree is the wave's part, over the
+// 256 values at sh; every lane of the wave returns the sum.
+__device__ __forceinline__ double block_tree(const double *sh) {
+  const int lane = threadIdx.x & (kWave - 1);
+  static_assert(kBlock == 4 * kWave, "two LDS levels");
+  return wave_sum((sh[lane] + sh[lane + 2 * kWave]) + (sh[lane + kWave] + sh[lane + 3 * kWave]));
+}
 __device__ __forceinline__ double block_sum(double v, double *sh) {
   const int tid = threadIdx.x;
   sh[tid] = v;
   __syncthreads();
-#pragma unroll
-  for (int off = kBlock / 2; off > 0; off >>= 1) {
-    if (tid < off) sh[tid] += sh[tid + off];
-    __syncthreads();
+  if (tid < kWave) {
+    const double r = block_tree(sh);
+    if (tid == 0) sh[0] = r;
   }
+  __syncthreads();
   const double r = sh[0];
   __syncthreads();
   return r;
@@ -808,69 +829,165 @@ __global__ __launch_bounds__(kBlock) void lowrank_stage_kernel(const R *X, int K
   if constexpr (NEXT) lr_write_partials<KT>(acc, K, part_out);
 }
 
+// r = sqrt((X/N)^2 + (Y/N)^2) in the working precision (kuramoto.cu:220:
+// pow((X/N*X/N + Y/N*Y/N), 0.5) with X, Y the sums of cos and sin).
+template <class R> __device__ __forceinline__ R order_value(double X, double Y, long N) {
+  const R XR = (R)X, YR = (R)Y, NR = (R)N;
+  return (R)pow((double)(XR / NR * XR / NR + YR / NR * YR / NR), 0.5);
+}
+
+// Order parameters of n emitted rows from their workgroups' partial sums
+// (nblk pairs a row), one wave per row: the sum over partials b, b + 256, ...
+// of each b < 256, then block_tree's order.
+template <class R>
+__device__ __forceinline__ void order_rows(int n, const double *part, int nblk, long N, R *r) {
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  for (int q = wave; q < n; q += kBlock / kWave) {
+    const double2 *p = reinterpret_cast<const double2 *>(part) + (size_t)q * nblk;
+    double x[4] = {0, 0, 0, 0}, y[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      for (int b = lane + v * kWave; b < nblk; b += kBlock) {
+        const double2 e = p[b];
+        x[v] += e.x;
+        y[v] += e.y;
+      }
+    const double X = wave_sum((x[0] + x[2]) + (x[1] + x[3]));
+    const double Y = wave_sum((y[0] + y[2]) + (y[1] + y[3]));
+    if (lane == 0) r[q] = order_value<R>(X, Y, N);
+  }
+}
+
 // ---------------------------------------------------------------------
-// Controller (dp45.cu:117-138): one workgroup.
+// Controller (dp45.cu:117-138): one workgroup, bound by the latency of its
+// chain of loads and of the norm's pow.  The state is read once at the start
+// (with the error partials in flight beside it), the decision is taken by
+// every lane of wave 0 in registers with the next 64 output times already
+// loaded, and written back once.
 // ---------------------------------------------------------------------
 template <class R>
 __global__ __launch_bounds__(kBlock) void control_kernel(State<R> *st, const double *err_part, int nparts, long N,
-                                                         const R *t_eval, R *times) {
-  if (!st->active || st->commit_pending) return;
+                                                         const R *t_eval, R *times, const double *ord_part, int nblk,
+                                                         R *r_ring) {
   __shared__ double sh[kBlock];
   double s = 0.0;
+#pragma unroll 8
   for (int b = threadIdx.x; b < nparts; b += kBlock) s += err_part[b];
-  const double sum = block_sum(s, sh);
-  if (threadIdx.x != 0) return;
-  st->attempts += 1;
-  st->rhs_evals += 6;
-  const R t = st->t;
-  R h = st->h;
-  int accept;
-  R hnext = h;
-  if (st->fixed) {
-    accept = 1;
-  } else {
-    const R nrm = (R)sqrt(sum);                                // {S,D}nrm2
-    const R norm = (R)((double)nrm / sqrt((double)N));        // dp45.cu:119
-    R factor = (R)(0.9 * pow((double)norm, -0.2));            // dp45.cu:120
-    st->norm = (double)norm;
-    if (norm < (R)1) {
+  sh[threadIdx.x] = s;
+  const State<R> S = *st;
+  const int lane = threadIdx.x % kWave;
+  const int e0 = S.commit_pending ? S.pend_lo : S.eval_i;
+  R te = e0 + lane < S.n_eval ? t_eval[e0 + lane] : (R)NAN;  // NaN: never reached
+  if (S.fin_n > 0)  // the previous attempt's rows
+    order_rows<R>(S.fin_n, ord_part + (size_t)S.job_slot * nblk * 2, nblk, N, r_ring + S.job_slot);
+  __syncthreads();
+  if (threadIdx.x >= kWave) return;
+  int active = S.active, pending = S.commit_pending, lo = S.pend_lo, hi = S.pend_hi;
+  int mode = JOB_NONE, n_emit = 0;
+  R tn = S.t;
+  if (active && !pending) {
+    const R h = S.h;
+    int accept, error = 0;
+    R hnext = h;
+    double norm_d = S.norm;
+    if (S.fixed) {
       accept = 1;
-      if (factor > (R)10) factor = (R)10;
-      hnext = h * factor;
     } else {
-      accept = 0;
-      if (factor < (R)1) {
-        if ((double)factor < 0.2) factor = (R)0.2;
+      const R nrm = (R)sqrt(block_tree(sh));                     // {S,D}nrm2
+      const R norm = (R)((double)nrm / sqrt((double)N));        // dp45.cu:119
+      R factor = (R)(0.9 * pow((double)norm, -0.2));            // dp45.cu:120
+      norm_d = (double)norm;
+      if (norm < (R)1) {
+        accept = 1;
+        if (factor > (R)10) factor = (R)10;
         hnext = h * factor;
+      } else {
+        accept = 0;
+        if (factor < (R)1) {
+          if ((double)factor < 0.2) factor = (R)0.2;
+          hnext = h * factor;
+        }
+        if (isnan((double)norm)) {  // the reference would loop forever here
+          error = 1;
+          active = 0;
+        }
       }
-      if (isnan((double)norm)) {  // the reference would loop forever here
-        st->error = 1;
-        st->active = 0;
+    }
+    if (accept) {
+      tn = S.t + h;
+      // output times crossed by this step (kuramoto.cu:205-212): up to the
+      // first one not reached
+      lo = S.eval_i;
+      hi = lo;
+      for (;;) {
+        const unsigned long long miss = ~__ballot(tn >= te);
+        hi += miss ? __ffsll((long long)miss) - 1 : kWave;
+        if (miss) break;
+        te = hi + lane < S.n_eval ? t_eval[hi + lane] : (R)NAN;
+      }
+      pending = 1;
+    } else {
+      mode = active ? JOB_STAGE2 : JOB_NONE;
+    }
+    if (lane == 0) {
+      st->attempts = S.attempts + 1;
+      st->rhs_evals = S.rhs_evals + 6;
+      st->norm = norm_d;
+      st->last_accept = accept;
+      st->h = hnext;
+      if (accept) {
+        st->t_last = S.t;
+        st->t = tn;
+        st->accepted = S.accepted + 1;
+        if (S.times_count < S.times_cap) {
+          times[2 * S.times_count] = tn;
+          times[2 * S.times_count + 1] = hnext;
+          st->times_count = S.times_count + 1;
+        }
+      } else {
+        st->rejected = S.rejected + 1;
+        if (error) {
+          st->error = 1;
+          st->active = 0;
+        }
       }
     }
   }
-  st->last_accept = accept;
-  if (!accept) {
-    st->rejected += 1;
-    st->h = hnext;
-    return;
+  if (active && pending) {
+    const int room = S.ring_cap - S.ring_count;
+    n_emit = hi - lo < room ? hi - lo : room;
+    const bool all = n_emit == hi - lo;
+    mode = all ? JOB_COMMIT : JOB_EMIT;
+    if (lane == 0) {
+      st->job_lo = lo;
+      st->job_slot = S.ring_count;
+      st->ring_count = S.ring_count + n_emit;
+      st->pend_lo = lo + n_emit;
+      st->pend_hi = hi;
+      st->commit_pending = all ? 0 : 1;
+      if (all) {
+        st->eval_i = hi;
+        if (!(tn < S.t1)) st->active = 0;
+      }
+    }
   }
-  const R tn = t + h;
-  st->t_last = t;
-  st->t = tn;
-  st->h = hnext;
-  st->accepted += 1;
-  if (st->times_count < st->times_cap) {
-    times[2 * st->times_count] = tn;
-    times[2 * st->times_count + 1] = hnext;
-    st->times_count += 1;
+  if (lane == 0) {
+    st->job_mode = mode;
+    st->job_n = n_emit;
+    st->fin_n = n_emit;
   }
-  // output times crossed by this step (kuramoto.cu:205-212)
-  int j = st->eval_i;
-  while (j < st->n_eval && tn >= t_eval[j]) ++j;
-  st->pend_lo = st->eval_i;
-  st->pend_hi = j;
-  st->commit_pending = 1;
+}
+
+// The order parameters control_kernel has not computed yet (after the last
+// attempt before the host reads the ring).
+template <class R>
+__global__ __launch_bounds__(kBlock) void finalize_kernel(State<R> *st, const double *ord_part, int nblk, long N,
+                                                          R *r_ring) {
+  const int n = st->fin_n, slot = st->job_slot;
+  if (n <= 0) return;
+  order_rows<R>(n, ord_part + (size_t)slot * nblk * 2, nblk, N, r_ring + slot);
+  __syncthreads();
+  if (threadIdx.x == 0) st->fin_n = 0;
 }
 
 // ---------------------------------------------------------------------
@@ -913,100 +1030,81 @@ template <class R> __device__ __forceinline__ void stage2_vector(const EmitArgs<
   a.cs_out[a.ldv + i] = s;
 }
 
+// n output rows of one dense-output interval: te(q) the q-th output time,
+// put(q, value) keeps this thread's value, part(q) the row's partial sums of
+// this workgroup.  Four rows at a time: their cos / sin, then one wave sums
+// each row (block_tree), so a group of rows costs two barriers and one chain
+// of latencies (one row at a time: 12 rows of N = 10^4 took 21 us).
+constexpr int kEmitRows = kBlock / kWave;
+template <class R, class TE, class PUT, class PART>
+__device__ __forceinline__ void emit_rows(int n, bool valid, const R Q[4], R yl, R tl, R hh,
+                                          double (&sh)[kEmitRows][2][kBlock], TE te, PUT put, PART part) {
+  const int tid = threadIdx.x, wave = tid / kWave;
+  for (int q0 = 0; q0 < n; q0 += kEmitRows) {
+    const int m = n - q0 < kEmitRows ? n - q0 : kEmitRows;
+#pragma unroll
+    for (int r = 0; r < kEmitRows; ++r) {
+      if (r >= m) break;
+      R c = 0, s = 0;
+      if (valid) {
+        const R x = (te(q0 + r) - tl) / hh;
+        const R val = dense_value<R>(Q, yl, hh, x);
+        put(q0 + r, val);
+        rsincos<R>(val, c, s);
+      }
+      sh[r][0][tid] = (double)c;
+      sh[r][1][tid] = (double)s;
+    }
+    __syncthreads();
+    if (wave < m) {
+      const double bc = block_tree(sh[wave][0]), bs = block_tree(sh[wave][1]);
+      if (tid % kWave == 0) *part(q0 + wave) = make_double2(bc, bs);
+    }
+    __syncthreads();
+  }
+}
+
 template <class R>
 __global__ __launch_bounds__(kBlock) void emit_commit_kernel(const EmitArgs<R> a) {
   const State<R> *st = a.st;
-  if (!st->active) return;
-  __shared__ double sh[kBlock];
+  const int mode = st->job_mode;
+  if (mode == JOB_NONE) return;
+  __shared__ double sh[kEmitRows][2][kBlock];
   const long i = (long)blockIdx.x * kBlock + threadIdx.x;
   const bool valid = i < a.N;
   const R h = st->h;
-  if (!st->commit_pending) {
+  if (mode == JOB_STAGE2) {
     if (valid) stage2_vector<R>(a, i, a.y[i], a.k[0][i], h);
     return;
   }
-  const int pend = st->pend_hi - st->pend_lo;
-  const int room = st->ring_cap - st->ring_count;
-  const int n_emit = pend < room ? pend : room;
+  // every operand of the commit is in flight before the outputs are formed
+  R yo = 0, yn = 0, k7 = 0;
+  if (valid) yo = a.y[i], yn = a.ynew[i], k7 = a.k[6][i];
+  const int n_emit = st->job_n, slot0 = st->job_slot, lo = st->job_lo;
   if (n_emit > 0) {
-    const R t = st->t, tl = st->t_last;
-    const R hh = t - tl;
+    const R tl = st->t_last, hh = st->t - tl;
     R Q[4] = {0, 0, 0, 0};
-    R yl = 0;
     if (valid) {
       R kv[7];
 #pragma unroll
       for (int j = 0; j < 7; ++j) kv[j] = a.k[j][i];
       dense_coeffs<R>(kv, Q);
-      yl = a.y[i];
     }
-    for (int q = 0; q < n_emit; ++q) {
-      const int slot = st->ring_count + q;
-      const R te = a.t_eval[st->pend_lo + q];
-      const R x = (te - tl) / hh;
-      double cx = 0.0, sx = 0.0;
-      if (valid) {
-        const R val = dense_value<R>(Q, yl, hh, x);
-        if (a.ring) a.ring[(size_t)slot * a.ldv + i] = val;
-        R c, s;
-        rsincos<R>(val, c, s);
-        cx = (double)c;
-        sx = (double)s;
-      }
-      const double bc = block_sum(cx, sh);
-      const double bs = block_sum(sx, sh);
-      if (threadIdx.x == 0) {
-        a.ord_part[((size_t)slot * gridDim.x + blockIdx.x) * 2] = bc;
-        a.ord_part[((size_t)slot * gridDim.x + blockIdx.x) * 2 + 1] = bs;
-      }
-    }
+    emit_rows<R>(
+        n_emit, valid, Q, yo, tl, hh, sh, [&](int q) { return a.t_eval[lo + q]; },
+        [&](int q, R val) {
+          if (a.ring) a.ring[(size_t)(slot0 + q) * a.ldv + i] = val;
+        },
+        [&](int q) {
+          return reinterpret_cast<double2 *>(a.ord_part) + (size_t)(slot0 + q) * gridDim.x + blockIdx.x;
+        });
   }
-  if (n_emit == pend && valid) {
+  if (mode == JOB_COMMIT && valid) {
     // commit (dp45.cu:123-125, FSAL copy :160) and the next stage-2 vector
-    const R yo = a.y[i], yn = a.ynew[i], k7 = a.k[6][i];
     a.ylast[i] = yo;
     a.y[i] = yn;
     a.k[0][i] = k7;
     stage2_vector<R>(a, i, yn, k7, h);
-  }
-}
-
-// r = sqrt((X/N)^2 + (Y/N)^2) in the working precision (kuramoto.cu:220:
-// pow((X/N*X/N + Y/N*Y/N), 0.5) with X, Y the sums of cos and sin).
-template <class R> __device__ __forceinline__ R order_value(double X, double Y, long N) {
-  const R XR = (R)X, YR = (R)Y, NR = (R)N;
-  return (R)pow((double)(XR / NR * XR / NR + YR / NR * YR / NR), 0.5);
-}
-
-template <class R>
-__global__ __launch_bounds__(kBlock) void finalize_kernel(State<R> *st, const double *ord_part, int nblk, long N,
-                                                          R *r_ring) {
-  if (!st->active || !st->commit_pending) return;
-  __shared__ double sh[kBlock];
-  const int pend = st->pend_hi - st->pend_lo;
-  const int room = st->ring_cap - st->ring_count;
-  const int n_emit = pend < room ? pend : room;
-  const int base = st->ring_count;
-  for (int q = 0; q < n_emit; ++q) {
-    const int slot = base + q;
-    double sx = 0, sy = 0;
-    for (int b = threadIdx.x; b < nblk; b += kBlock) {
-      sx += ord_part[((size_t)slot * nblk + b) * 2];
-      sy += ord_part[((size_t)slot * nblk + b) * 2 + 1];
-    }
-    const double X = block_sum(sx, sh);
-    const double Y = block_sum(sy, sh);
-    if (threadIdx.x == 0) r_ring[slot] = order_value<R>(X, Y, N);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    st->ring_count = base + n_emit;
-    st->pend_lo += n_emit;
-    if (st->pend_lo == st->pend_hi) {
-      st->commit_pending = 0;
-      st->eval_i = st->pend_hi;
-      if (!(st->t < st->t1)) st->active = 0;
-    }
   }
 }
 
