@@ -174,6 +174,38 @@ template <class T> __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
+// The NV values v[0..NV) of every lane, each summed over the wave in
+// wave_sum's order (the same bits): lane l returns the sum of value
+// wave_slot<NV>(l).  At each distance half of the remaining values go to the
+// partner lane, so NV = 16 takes 8 + 4 + 2 + 1 + 1 + 1 exchanges instead of
+// 16 x 6.
+template <int NV> __device__ __forceinline__ int wave_slot(int lane) {
+  int slot = 0;
+#pragma unroll
+  for (int half = NV / 2, off = kWave / 2; half > 0; half /= 2, off /= 2) slot += (lane & off) ? half : 0;
+  return slot;
+}
+template <class T, int HALF, int OFF, int NV> __device__ __forceinline__ T wave_reduce_from(T (&v)[NV], int lane) {
+  if constexpr (HALF > 0) {
+    const bool up = lane & OFF;
+#pragma unroll
+    for (int k = 0; k < HALF; ++k) {
+      const T keep = up ? v[k + HALF] : v[k], send = up ? v[k] : v[k + HALF];
+      v[k] = keep + __shfl_xor(send, OFF, kWave);
+    }
+    return wave_reduce_from<T, HALF / 2, OFF / 2>(v, lane);
+  } else {
+    T s = v[0];
+#pragma unroll
+    for (int off = OFF; off > 0; off >>= 1) s += __shfl_xor(s, off, kWave);
+    return s;
+  }
+}
+template <class T, int NV> __device__ __forceinline__ T wave_reduce(T (&v)[NV], int lane) {
+  static_assert(NV >= 1 && NV <= kWave && (NV & (NV - 1)) == 0, "a power of two");
+  return wave_reduce_from<T, NV / 2, kWave / 2>(v, lane);
+}
+
 // Deterministic sum of one double per thread of a workgroup, in a fixed tree:
 // x[t] + x[t + 128], then + 64, 32, ... 1.  The first two levels are read
 // from LDS by one wave, the others are lane exchanges (a barrier per level
@@ -228,13 +260,39 @@ template <class R> __device__ __forceinline__ R rhs_value(R om, R c1, R cs, R sn
   return rfma<R>(c1, rfma<R>(sn, C, -(cs * S)), om);
 }
 
+// What the row epilogue of oscillator i reads besides C and S.  Loaded on
+// its own so that kernels can have these loads in flight while they reduce
+// the coupling sums (a dependent load costs 1-2 us between short kernels).
+template <class R, int KIND> struct RowOps {
+  static constexpr int NK = KIND >= 2 ? KIND - 1 : 0;  // k_1 .. k_{s-1}
+  R cs, sn, om, y, yn, h, atl, rtl;
+  R k[NK > 0 ? NK : 1];
+};
+template <class R, int KIND> __device__ __forceinline__ RowOps<R, KIND> row_load(const Vecs<R> &a, long i) {
+  RowOps<R, KIND> o;
+  o.cs = a.cs_in[i];
+  o.sn = a.cs_in[a.ldv + i];
+  o.om = a.omega[i];
+  if constexpr (KIND >= 2) {
+#pragma unroll
+    for (int j = 0; j < KIND - 1; ++j) o.k[j] = a.k[j][i];
+    o.y = a.y[i];
+    o.h = a.st->h;
+  }
+  if constexpr (KIND == 7) {
+    o.yn = a.ynew[i];
+    o.rtl = a.st->rtl;
+    o.atl = a.st->atl;
+  }
+  return o;
+}
+
 // Row epilogue for oscillator i.  Returns the squared scaled error of
 // stage 7 (0 otherwise).  Stage combinations follow dp45.cu:34-69 with the
 // contraction acc = k1*a0; acc = fma(k_j, a_j, acc); y + h*acc -> fma(acc, h, y).
 template <class R, int KIND>
-__device__ __forceinline__ double row_epilogue(const Vecs<R> &a, long i, R C, R S, R h) {
-  const R cs = a.cs_in[i], sn = a.cs_in[a.ldv + i];
-  const R f = rhs_value<R>(a.omega[i], a.c1, cs, sn, C, S);
+__device__ __forceinline__ double row_finish(const Vecs<R> &a, long i, const RowOps<R, KIND> &o, R C, R S) {
+  const R f = rhs_value<R>(o.om, a.c1, o.cs, o.sn, C, S);
   if constexpr (KIND == KIND_RHS) {
     a.f_out[i] = f;
     if (a.cs_pairs) { a.cs_pairs[2 * i] = C; a.cs_pairs[2 * i + 1] = S; }
@@ -248,13 +306,10 @@ __device__ __forceinline__ double row_epilogue(const Vecs<R> &a, long i, R C, R 
     a.k[s - 1][i] = f;
     if constexpr (s < 7) {
       // coefficients of stage s+1 over k_1..k_s
-      R acc = a.k[0][i] * (R)tab::A[s - 1][0];
+      R acc = o.k[0] * (R)tab::A[s - 1][0];
 #pragma unroll
-      for (int j = 1; j < s; ++j) {
-        const R kj = (j == s - 1) ? f : a.k[j][i];
-        acc = rfma<R>(kj, (R)tab::A[s - 1][j], acc);
-      }
-      const R yt = rfma<R>(acc, h, a.y[i]);
+      for (int j = 1; j < s; ++j) acc = rfma<R>(j == s - 1 ? f : o.k[j < s - 1 ? j : 0], (R)tab::A[s - 1][j], acc);
+      const R yt = rfma<R>(acc, o.h, o.y);
       if constexpr (s + 1 == 7) a.ynew[i] = yt;
       R c, sn1;
       rsincos<R>(yt, c, sn1);
@@ -263,19 +318,19 @@ __device__ __forceinline__ double row_epilogue(const Vecs<R> &a, long i, R C, R 
       return 0.0;
     } else {
       // embedded error, dp45.cu:79-84
-      R acc = a.k[0][i] * (R)tab::E[0];
+      R acc = o.k[0] * (R)tab::E[0];
 #pragma unroll
-      for (int j = 1; j < 7; ++j) {
-        const R kj = (j == 6) ? f : a.k[j][i];
-        acc = rfma<R>(kj, (R)tab::E[j], acc);
-      }
-      const R st = a.st->rtl;
-      const R num = h * acc;
-      const R den = rfma<R>(st, rmax<R>(rabs<R>(a.y[i]), rabs<R>(a.ynew[i])), a.st->atl);
+      for (int j = 1; j < 7; ++j) acc = rfma<R>(j == 6 ? f : o.k[j < 6 ? j : 0], (R)tab::E[j], acc);
+      const R num = o.h * acc;
+      const R den = rfma<R>(o.rtl, rmax<R>(rabs<R>(o.y), rabs<R>(o.yn)), o.atl);
       const R e = num / den;
       return (double)e * (double)e;
     }
   }
+}
+template <class R, int KIND>
+__device__ __forceinline__ double row_epilogue(const Vecs<R> &a, long i, R C, R S) {
+  return row_finish<R, KIND>(a, i, row_load<R, KIND>(a, i), C, S);
 }
 
 // ---------------------------------------------------------------------
@@ -292,9 +347,10 @@ template <class R, class S> struct DenseArgs {
   Vecs<R> v;
 };
 
-// Row sums of one group of ROWS rows [row0, row_end): wave shuffles, then
-// the 4 wave sums in wave order (fixed tree), scale, row epilogue.  Returns
-// (in thread 0) the group's sum of squared scaled errors for stage 7.
+// Row sums of one group of ROWS rows [row0, row_end): the wave sums
+// (wave_reduce), then the 4 wave sums in wave order (fixed tree), scale, row
+// epilogue, its operands loaded before the reduction.  Returns (in thread 0)
+// the group's sum of squared scaled errors for stage 7.
 template <class R, class Acc, int ROWS, int KIND>
 __device__ __forceinline__ double finish_group(Acc (&accC)[ROWS], Acc (&accS)[ROWS], long row0, long row_end,
                                                R mscale, const Vecs<R> &v) {
@@ -302,25 +358,23 @@ __device__ __forceinline__ double finish_group(Acc (&accC)[ROWS], Acc (&accS)[RO
   __shared__ double errsq[ROWS];
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1), wave = tid / kWave;
+  const long i = row0 + tid;
+  // every lane loads (a row it shares with others): no branch around loads
+  const long il = row0 + tid % ROWS;
+  const RowOps<R, KIND> ops = row_load<R, KIND>(v, il < row_end ? il : row_end - 1);
+  Acc val[2 * ROWS];
 #pragma unroll
-  for (int r = 0; r < ROWS; ++r) {
-    accC[r] = wave_sum(accC[r]);
-    accS[r] = wave_sum(accS[r]);
-  }
-  if (lane == 0) {
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r) { red[wave][r] = accC[r]; red[wave][ROWS + r] = accS[r]; }
-  }
+  for (int r = 0; r < ROWS; ++r) { val[r] = accC[r]; val[ROWS + r] = accS[r]; }
+  const Acc tot = wave_reduce<Acc, 2 * ROWS>(val, lane);
+  red[wave][wave_slot<2 * ROWS>(lane)] = tot;  // the lanes of a slot hold the same sum
   __syncthreads();
   if (tid < ROWS) {
-    const long i = row0 + tid;
     double sq = 0.0;
     if (i < row_end) {
       Acc C = red[0][tid], Sv = red[0][ROWS + tid];
 #pragma unroll
       for (int w = 1; w < kBlock / kWave; ++w) { C += red[w][tid]; Sv += red[w][ROWS + tid]; }
-      const R h = (KIND >= 2) ? v.st->h : (R)0;
-      sq = row_epilogue<R, KIND>(v, i, (R)C * mscale, (R)Sv * mscale, h);
+      sq = row_finish<R, KIND>(v, i, ops, (R)C * mscale, (R)Sv * mscale);
     }
     if constexpr (KIND == 7) errsq[tid] = sq;
   }
@@ -681,8 +735,7 @@ __global__ __launch_bounds__(kBlock) void lowrank_expand_kernel(const R *X, int 
       C = __builtin_fma(x, G[2 * m], C);
       S = __builtin_fma(x, G[2 * m + 1], S);
     }
-    const R h = (KIND >= 2) ? v.st->h : (R)0;
-    sq = row_epilogue<R, KIND>(v, i, (R)C, (R)S, h);
+    sq = row_epilogue<R, KIND>(v, i, (R)C, (R)S);
   }
   if constexpr (KIND == 7) {
     const double tot = block_sum(sq, errsq);
@@ -799,7 +852,6 @@ __global__ __launch_bounds__(kBlock) void lowrank_stage_kernel(const R *X, int K
   double acc[2 * KT];
 #pragma unroll
   for (int q = 0; q < 2 * KT; ++q) acc[q] = 0.0;
-  const R h = (KIND >= 2) ? v.st->h : (R)0;
   double sq = 0.0;
   for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < v.N; i += (long)gridDim.x * kBlock) {
     double x[KT];
@@ -811,7 +863,7 @@ __global__ __launch_bounds__(kBlock) void lowrank_stage_kernel(const R *X, int K
         C = __builtin_fma(x[m], g[2 * m], C);
         S = __builtin_fma(x[m], g[2 * m + 1], S);
       }
-    sq += row_epilogue<R, KIND>(v, i, (R)C, (R)S, h);
+    sq += row_epilogue<R, KIND>(v, i, (R)C, (R)S);
     if constexpr (NEXT) {
       const double c = v.cs_out[i], s = v.cs_out[v.ldv + i];
 #pragma unroll

@@ -389,8 +389,7 @@ __global__ __launch_bounds__(kBlock) void sign_stage_kernel(const int32_t *__res
       C = sign_combine(sc);
       S = sign_combine(ss);
     }
-    const R h = (KIND >= 2) ? v.st->h : (R)0;
-    sq = row_epilogue<R, KIND>(v, i, (R)C, (R)S, h);
+    sq = row_epilogue<R, KIND>(v, i, (R)C, (R)S);
   }
   if constexpr (KIND == 7) {
     const double tot = block_sum(sq, errsq);

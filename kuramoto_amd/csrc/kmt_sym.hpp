@@ -328,8 +328,7 @@ __global__ __launch_bounds__(kBlock) void sym_reduce_kernel(const SymArgs<R, S> 
       C += p.c;
       Sn += p.s;
     }
-    const R h = (KIND >= 2) ? a.v.st->h : (R)0;
-    sq = row_epilogue<R, KIND>(a.v, i, (R)C * a.mscale, (R)Sn * a.mscale, h);
+    sq = row_epilogue<R, KIND>(a.v, i, (R)C * a.mscale, (R)Sn * a.mscale);
   }
   if constexpr (KIND == 7) {
     const double s = block_sum(sq, sh);
