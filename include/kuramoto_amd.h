@@ -233,10 +233,12 @@ int kmt_bandwidth_probe(int device, size_t bytes, int reps, double *copy_gbps, d
  * Every row is summed in the same order in every variant; the error norm's
  * partial sums follow the variant's workgroups (the ring groups them as the
  * loop without it does), so its last bits (and h's) can differ between
- * variants.  Without this call kmt_begin uses a fixed choice (4 rows, plain
- * loads when N >= 4096 and the matrix is <= 128 MB; else 8 rows, 16 for
- * 16-bit entries, non-temporal; the chunk ring unless the entries are 16
- * bits), so that every context and process gives the same bits.
+ * variants.  Without this call a fixed choice is used (a matrix of up to
+ * 256 MB: plain loads, 4 rows, 8 for N < 4096 and for 16-bit entries with
+ * FP64 state; a larger one: non-temporal loads, 8 rows, 16 for 16-bit
+ * entries with FP64 state or N >= 50000; the chunk ring for the working precision, and for 16-bit entries
+ * of up to 256 MB with FP32 state), so that every context and process gives
+ * the same bits.
  * Calling it (mid-run, or in only one of two contexts) therefore breaks
  * bit-exact restart against contexts that use the fixed choice.  KMT_ADJ_SYM has one
  * form and is not tuned.  No reference counterpart (cuBLAS chooses its own

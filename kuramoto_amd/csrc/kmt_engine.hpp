@@ -212,28 +212,47 @@ template <class R> struct Engine : EngineBase {
   // and with it the last bits of the error norm and of h, follows the
   // variant.  kmt_begin therefore picks it by a fixed rule, not by timing,
   // so that runs and restarts of one problem give the same bits in every
-  // context and process: from N = 4096 on, a matrix that fits the 256 MB
-  // Infinity Cache twice over takes 4 rows per group with plain loads, a
-  // larger one 8 rows with non-temporal loads (the autotuner's picks at
-  // N=5000 FP32 and N=50000 FP32/FP64); smaller N keep 8 rows, the grouping
-  // of the FP64 register-rebuild kernel.  A larger 16-bit matrix takes 16
-  // rows: each (cos, sin) chunk is reused for every row of the group from
-  // registers, and at 8 rows the vectors' L2 bytes would match the 2-byte
-  // entries' (FP64 state, BF16, N=50000: 0.754 against 0.811 ms per stage).
-  // A matrix in the working precision takes the chunk ring (the same sums
-  // and grouping; 0.6% faster at N=50000 FP64 and FP32 from HBM, 4.4% at
-  // N=5000 FP32 from the Infinity Cache; slower with 16-bit entries at 16
-  // rows, where it needs 231 registers).
+  // context and process.
+  //  * A matrix that fits the 256 MB Infinity Cache is read from it by every
+  //    stage after the first, so its loads are plain (a non-temporal load
+  //    does not keep the line: FP64 N=5000, 200 MB, 34.8 -> 30.6 us; FP32
+  //    N=8000, 256 MB, 40.6 -> 38.1; BF16 N=11000, 242 MB, 43.6 -> 36.7; from
+  //    484 MB on plain loads lose: FP32 N=11000 83.8 against 74.0), and from
+  //    N = 4096 on it takes 4 rows per group, which fills the chip at N=5000
+  //    (17.8 against 18.2 us with 8 rows, 20.9 with 16).  With FP64 vectors
+  //    and 16-bit entries 8 rows: the vectors' bytes are then no more than the
+  //    entries' (BF16 N=8000: 26.1 us against 30.7 with 4 rows).  Smaller N
+  //    keep 8 rows, the grouping of the FP64 register-rebuild kernel.
+  //  * A larger one takes 8 rows with non-temporal loads, 16 rows with 16-bit
+  //    entries (each (cos, sin) chunk is reused for every row of the group:
+  //    FP64 state, BF16, N=50000: 0.752 against 0.812 ms with 8 rows; FP32
+  //    state, FP16, N=200000: 11.4 against 12.0), but 8 with FP32 vectors
+  //    below N = 50000, where the vectors are small and the shorter groups end
+  //    more evenly (BF16 N=14000: 62.8 against 65.2 us; N=50000: level).
+  //  * The chunk ring wherever it measured faster: the working precision
+  //    (0.6% at N=50000, 2-4% from the cache) and 16-bit entries with FP32
+  //    vectors from the cache (5%); with 16 rows of 16-bit entries it needs
+  //    231 registers and is 5% slower.
   // kmt_autotune / kmt_select_variant override it.
   void default_variant() {
-    const bool cached = N >= 4096 && (double)N * (double)N * (double)elem_bytes(storage) <= 128e6;
-    tune_rows = cached ? 4 : (elem_bytes(storage) == 2 ? 16 : 8);
+    const bool half = elem_bytes(storage) == 2;
+    const bool cached = (double)N * (double)N * (double)elem_bytes(storage) <= 256e6;
+    tune_rows = !cached ? (half && (sizeof(R) == 8 || N >= 50000) ? 16 : 8) : N < 4096 || (half && sizeof(R) == 8) ? 8 : 4;
     tune_nt = cached ? 0 : 1;
     tune_bal = 0;
-    tune_ring = elem_bytes(storage) != 2;
+    tune_ring = !half || (cached && sizeof(R) == 4);
     bal_grid = 0;
     tuned = 1;
     drop_graphs();
+  }
+
+  // Every entry point that launches the dense kernel uses the rule's choice:
+  // a right-hand side evaluated before any run too (it used to take 8 rows
+  // without the ring whatever the storage: FP64 state, BF16, N=50000 0.802 ms
+  // against 0.757 with 16 rows).  Rows are summed in the same order in every
+  // variant.  No HIP call when there is nothing to drop: safe under capture.
+  void ensure_variant() {
+    if (!tuned && !factored && !sym()) default_variant();
   }
 
   int select_variant(int rows, int flags) override {
@@ -1104,6 +1123,7 @@ template <class R> struct Engine : EngineBase {
   // ---------------- model evaluations ----------------
   int rhs(const void *th, void *f, void *cpl) override {
     if (!coupling_ready()) return fail(KMT_ERR_STATE, "no adjacency: call kmt_set_adjacency, kmt_build_adjacency or kmt_set_factor + kmt_use_factored");
+    ensure_variant();
     HIP_TRY(hipMemcpyAsync(vec_scr, th, sizeof(R) * N, hipMemcpyHostToDevice, stream));
     sincos_kernel<R><<<(unsigned)((N + kBlock - 1) / kBlock), kBlock, 0, stream>>>(vec_scr, N, ldv, cs_scr);
     Vecs<R> v = vecs(cs_scr, nullptr, 0);
@@ -1124,6 +1144,7 @@ template <class R> struct Engine : EngineBase {
   // allocated; the factored path uses the context's partial-sum buffers.
   int rhs_device(const void *th, void *f, void *cpl, void *cs, hipStream_t s) override {
     if (!coupling_ready()) return fail(KMT_ERR_STATE, "no adjacency: call kmt_set_adjacency, kmt_build_adjacency or kmt_set_factor + kmt_use_factored");
+    ensure_variant();
     const hipStream_t own = stream;
     stream = s ? s : own;
     sincos_pad_kernel<R><<<(unsigned)((ldv + kBlock - 1) / kBlock), kBlock, 0, stream>>>((const R *)th, N, ldv, (R *)cs);
@@ -1192,7 +1213,7 @@ template <class R> struct Engine : EngineBase {
     shadow.rhs_evals = 1;
     shadow.job_mode = shadow.active ? JOB_STAGE2 : JOB_NONE;
     KMT_TRY(push_state());
-    if (!tuned && !factored && !sym()) default_variant();
+    ensure_variant();
     // k1 = f(y) (dp45.cu:151), then the first stage-2 vector
     sincos_kernel<R><<<(unsigned)((N + kBlock - 1) / kBlock), kBlock, 0, stream>>>(y, N, ldv, cs[1]);
     Vecs<R> v = vecs(cs[1], nullptr, 0);
@@ -1324,6 +1345,7 @@ template <class R> struct Engine : EngineBase {
   int time_stage(int reps, double *avg_ms) override {
     if (!coupling_ready()) return fail(KMT_ERR_STATE, "no adjacency");
     if (reps < 1) return fail(KMT_ERR_ARG, "reps < 1");
+    ensure_variant();
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
