@@ -11,6 +11,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/kuramoto_amd.h"
@@ -82,7 +83,7 @@ template <class R> struct Engine : EngineBase {
   void *A = nullptr;
   size_t A_bytes = 0;
   R *X = nullptr, *w = nullptr;
-  R *XT = nullptr;  // transposed factor [K][ldv] for the register-rebuild form
+  R *XT = nullptr;  // transposed factor [K][ldv] (K <= kLrMaxRank): the low-rank and register-rebuild forms
   int K = 0;
   int factored = 0;  // 0 dense A, KMT_LOWRANK_CONTRACT, KMT_LOWRANK_REBUILD
   // KMT_ADJ_SYM: (I, J) of each stored block, and the row / column partials
@@ -90,7 +91,7 @@ template <class R> struct Engine : EngineBase {
   int2 *sym_ij = nullptr;
   SymPair<double> *sym_prow = nullptr, *sym_pcol = nullptr;
   double *lr_part = nullptr, *lr_G = nullptr;
-  int lr_nblk = 0, lr_grid = 0;
+  int lr_nblk = 0, lr_grid = 0, lr_threads = kBlock;
   // packed +-1 factor (kmt_set_factor_sign): per pass (1: rows m over
   // k = n, 2: rows n over k = m) the sign bits in the pass's tile order
   // (ldp rows of 32 npairs words: the bit rows, the ones row, zero rows),
@@ -516,14 +517,24 @@ template <class R> struct Engine : EngineBase {
       HIP_TRY(hipMemcpyAsync(w, wv, sizeof(R) * K, hipMemcpyHostToDevice, stream));
     }
     lr_nblk = (int)std::min<long>((N + kBlock - 1) / kBlock, 512);
-    lr_grid = (int)std::min<long>((N + kBlock - 1) / kBlock, kLrMaxBlocks);
-    const int nparts = std::max(lr_nblk, 2 * lr_grid);
+    // one row per thread, the workgroups spread over the CUs once
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) cus = 1;
+    lr_threads = (int)std::min<long>(std::max<long>(round_up((N + cus - 1) / cus, kWave), kBlock),
+                                     lr_max_threads(sizeof(R), lr_rank_bound()));
+    lr_grid = (int)std::min<long>((N + lr_threads - 1) / lr_threads, kLrMaxBlocks);
+    const int nparts = std::max(lr_nblk, 3 * lr_grid);
+    if (K <= kLrMaxRank) {
+      KMT_TRY(alloc_vec(&XT, (long)kk * ldv));
+      transpose_factor_kernel<R><<<(unsigned)((N + kBlock - 1) / kBlock), kBlock, 0, stream>>>(X, K, N, ldv, XT);
+      HIP_TRY(hipGetLastError());
+    }
     HIP_TRY(hipMalloc((void **)&lr_part, sizeof(double) * 2 * kk * nparts));
     HIP_TRY(hipMemsetAsync(lr_part, 0, sizeof(double) * 2 * kk * nparts, stream));
     HIP_TRY(hipMalloc((void **)&lr_G, sizeof(double) * 2 * kk));
     HIP_TRY(hipMemsetAsync(lr_G, 0, sizeof(double) * 2 * kk, stream));
     HIP_TRY(hipStreamSynchronize(stream));
-    if (factored == KMT_LOWRANK_REBUILD) {  // keep the mode: transpose the new factor
+    if (factored == KMT_LOWRANK_REBUILD) {  // keep the mode, if the new rank allows it
       factored = KMT_LOWRANK_CONTRACT;
       return use_factored(KMT_LOWRANK_REBUILD);
     }
@@ -727,17 +738,8 @@ template <class R> struct Engine : EngineBase {
     if (on && !X && !sign) return fail(KMT_ERR_STATE, "-A needs kmt_set_factor or kmt_set_factor_sign first");
     if (on == KMT_LOWRANK_REBUILD && sign)
       return fail(KMT_ERR_ARG, "register-rebuilt tiles need a real factor (kmt_set_factor), not a packed sign factor");
-    if (on == KMT_LOWRANK_REBUILD) {
-      if (K > kLrMaxRank) return fail(KMT_ERR_ARG, "register-rebuilt tiles support K <= %d (K=%d)", kLrMaxRank, K);
-      if (!XT) {
-        std::vector<R> t((size_t)std::max(K, 1) * ldv, (R)0);
-        for (long i = 0; i < N; ++i)
-          for (int m = 0; m < K; ++m) t[(size_t)m * ldv + i] = X_host[(size_t)i * K + m];
-        HIP_TRY(hipMalloc((void **)&XT, sizeof(R) * t.size()));
-        HIP_TRY(hipMemcpyAsync(XT, t.data(), sizeof(R) * t.size(), hipMemcpyHostToDevice, stream));
-        HIP_TRY(hipStreamSynchronize(stream));
-      }
-    }
+    if (on == KMT_LOWRANK_REBUILD && K > kLrMaxRank)
+      return fail(KMT_ERR_ARG, "register-rebuilt tiles support K <= %d (K=%d)", kLrMaxRank, K);
     if (factored != on) drop_graphs();
     factored = on;
     return KMT_OK;
@@ -866,29 +868,55 @@ template <class R> struct Engine : EngineBase {
   }
 
   bool lr_fused() const { return K <= kLrMaxRank && !sign; }
-  // partial-sum buffers of the fused low-rank path (used alternately)
+  bool lr_path() const { return factored == KMT_LOWRANK_CONTRACT && lr_fused(); }
+  // partial-sum buffers of the fused low-rank path: 0 and 1 alternate between
+  // the stages of an attempt (0: also the stage-2 vector's, kept between
+  // attempts), 2 belongs to stand-alone right-hand sides
   double *lr_p(int which) const { return lr_part + (size_t)which * 2 * std::max(K, 1) * lr_grid; }
-
-  template <int KT> void launch_gram_t(const R *cs_in, int which, int check) {
-    lowrank_gram_kernel<R, KT><<<(unsigned)lr_grid, kBlock, 0, stream>>>(X, K, N, cs_in, ldv, lr_p(which), st, check);
+  LrArgs<R> lr_args(int pin, int pout) const {
+    LrArgs<R> l;
+    l.XT = XT;
+    l.w = w;
+    l.K = K;
+    l.part_in = lr_p(pin);
+    l.nparts = lr_grid;
+    l.part_out = lr_p(pout);
+    return l;
   }
-  void launch_gram(const R *cs_in, int which, int check) {
-    if (K <= 8) launch_gram_t<8>(cs_in, which, check);
-    else launch_gram_t<16>(cs_in, which, check);
+  // the rank bound of the kernels that lr_dispatch picks
+  int lr_rank_bound() const { return K <= 8 ? std::max(K, 1) : kLrMaxRank; }
+  // f(rank bound, exact) for this context's rank
+  template <class F> void lr_dispatch(F &&f) {
+    using std::integral_constant;
+    switch (K) {
+      case 0: f(integral_constant<int, 1>{}, std::false_type{}); break;
+      case 1: f(integral_constant<int, 1>{}, std::true_type{}); break;
+      case 2: f(integral_constant<int, 2>{}, std::true_type{}); break;
+      case 3: f(integral_constant<int, 3>{}, std::true_type{}); break;
+      case 4: f(integral_constant<int, 4>{}, std::true_type{}); break;
+      case 5: f(integral_constant<int, 5>{}, std::true_type{}); break;
+      case 6: f(integral_constant<int, 6>{}, std::true_type{}); break;
+      case 7: f(integral_constant<int, 7>{}, std::true_type{}); break;
+      case 8: f(integral_constant<int, 8>{}, std::true_type{}); break;
+      default: f(integral_constant<int, kLrMaxRank>{}, std::false_type{}); break;
+    }
   }
-  // stage KIND from the partials in lr_p(pin); with NEXT, the partials of
-  // its output vector into lr_p(pin ^ 1)
-  template <int KIND, int KT, bool NEXT> void launch_lr_stage_t(const Vecs<R> &v, int pin) {
-    lowrank_stage_kernel<R, KIND, KT, NEXT><<<(unsigned)lr_grid, kBlock, 0, stream>>>(X, K, lr_p(pin), lr_grid, w, v,
-                                                                                       lr_p(pin ^ 1));
+  void launch_gram(const R *cs_in, int pout) {
+    lr_dispatch([&](auto kt, auto exact) {
+      lowrank_gram_kernel<R, decltype(kt)::value, decltype(exact)::value>
+          <<<(unsigned)lr_grid, lr_threads, 0, stream>>>(lr_args(0, pout), N, cs_in, ldv);
+    });
   }
-  template <int KIND, bool NEXT> void launch_lr_stage(const Vecs<R> &v, int pin) {
-    if (K <= 8) launch_lr_stage_t<KIND, 8, NEXT>(v, pin);
-    else launch_lr_stage_t<KIND, 16, NEXT>(v, pin);
+  // stage KIND from the partials in lr_p(pin); stages 2..6 write those of
+  // their output vector into lr_p(pout)
+  template <int KIND> void launch_lr_stage(const Vecs<R> &v, int pin, int pout) {
+    lr_dispatch([&](auto kt, auto exact) {
+      lowrank_stage_kernel<R, KIND, decltype(kt)::value, decltype(exact)::value>
+          <<<(unsigned)lr_grid, lr_threads, 0, stream>>>(lr_args(pin, pout), v);
+    });
   }
-  // one attempt's six stages on the fused low-rank path: partials of the
-  // stage-2 vector, then one launch per stage that also writes the partials
-  // of the next stage's vector
+  // one attempt's six stages on the fused low-rank path, one launch each
+  // (the stage-2 vector's partials: the previous emit)
   void launch_lr_attempt(std::vector<std::pair<hipEvent_t, hipEvent_t>> *ev) {
     for (int s = 2; s <= 7; ++s) {
       const R *in = cs[(s - 2) & 1];
@@ -896,14 +924,13 @@ template <class R> struct Engine : EngineBase {
       Vecs<R> v = vecs(in, out, 1);
       const int pin = (s - 2) & 1;
       if (ev) (void)hipEventRecord((*ev)[0].first, stream);
-      if (s == 2) launch_gram(in, 0, 1);
       switch (s) {
-        case 2: launch_lr_stage<2, true>(v, pin); break;
-        case 3: launch_lr_stage<3, true>(v, pin); break;
-        case 4: launch_lr_stage<4, true>(v, pin); break;
-        case 5: launch_lr_stage<5, true>(v, pin); break;
-        case 6: launch_lr_stage<6, true>(v, pin); break;
-        default: launch_lr_stage<7, false>(v, pin); break;
+        case 2: launch_lr_stage<2>(v, pin, pin ^ 1); break;
+        case 3: launch_lr_stage<3>(v, pin, pin ^ 1); break;
+        case 4: launch_lr_stage<4>(v, pin, pin ^ 1); break;
+        case 5: launch_lr_stage<5>(v, pin, pin ^ 1); break;
+        case 6: launch_lr_stage<6>(v, pin, pin ^ 1); break;
+        default: launch_lr_stage<7>(v, pin, pin ^ 1); break;
       }
       if (ev) {
         (void)hipEventRecord((*ev)[0].second, stream);
@@ -941,8 +968,8 @@ template <class R> struct Engine : EngineBase {
       return;
     }
     if (lr_fused()) {
-      launch_gram(v.cs_in, 0, v.check_state && KIND >= 2);
-      launch_lr_stage<KIND, false>(v, 0);
+      launch_gram(v.cs_in, 2);
+      launch_lr_stage<KIND>(v, 2, 1);
       return;
     }
     const int tiles = std::max(1, (K + kRankTile - 1) / kRankTile);
@@ -1080,7 +1107,7 @@ template <class R> struct Engine : EngineBase {
   // One attempt: stages 2..7 (cs ping-pong 0->1->0->1->0->1), control,
   // emit/commit (writes stage-2 vector into cs[0]).
   void launch_attempt(std::vector<std::pair<hipEvent_t, hipEvent_t>> *ev = nullptr) {
-    if (factored == KMT_LOWRANK_CONTRACT && lr_fused()) launch_lr_attempt(ev);
+    if (lr_path()) launch_lr_attempt(ev);
     else for (int s = 2; s <= 7; ++s) {
       const R *in = cs[(s - 2) & 1];
       R *out = cs[(s - 1) & 1];
@@ -1092,16 +1119,33 @@ template <class R> struct Engine : EngineBase {
         ev->erase(ev->begin());
       }
     }
-    control_kernel<R><<<1, kBlock, 0, stream>>>(st, err_part, n_parts_stage7(), N, t_eval, times, ord_part, nblk_emit,
-                                                r_ring);
-    emit_commit_kernel<R><<<(unsigned)nblk_emit, kBlock, 0, stream>>>(emit_args());
+    control_kernel<R><<<1, kBlock, 0, stream>>>(st, err_part, n_parts_stage7(), N, t_eval, times, ord_part,
+                                                emit_blocks(), r_ring);
+    launch_emit();
+  }
+  // workgroups of the emit launch (partials per emitted row)
+  int emit_blocks() const { return lr_path() ? lr_grid : nblk_emit; }
+  void launch_emit() {
+    if (lr_path())
+      lr_dispatch([&](auto kt, auto exact) {
+        lowrank_emit_kernel<R, decltype(kt)::value, decltype(exact)::value>
+            <<<(unsigned)lr_grid, lr_threads, 0, stream>>>(emit_args(), lr_args(0, 0));
+      });
+    else
+      emit_commit_kernel<R><<<(unsigned)nblk_emit, kBlock, 0, stream>>>(emit_args());
+  }
+  // Before the first attempt after a change of coupling: the low-rank path's
+  // partials of the pending stage-2 vector
+  void launch_prepare() {
+    if (lr_path()) launch_gram(cs[0], 0);
   }
   // the order parameters of the last attempt's rows (earlier ones are
   // computed by the next attempt's control_kernel): before the host looks
-  void launch_finalize() { finalize_kernel<R><<<1, kBlock, 0, stream>>>(st, ord_part, nblk_emit, N, r_ring); }
+  void launch_finalize() { finalize_kernel<R><<<1, kBlock, 0, stream>>>(st, ord_part, emit_blocks(), N, r_ring); }
 
   int build_graphs() {
     drop_graphs();
+    launch_prepare();
     for (int which = 0; which < 2; ++which) {
       const int n = which == 0 ? 1 : 8;
       hipGraph_t g = nullptr;
@@ -1219,7 +1263,7 @@ template <class R> struct Engine : EngineBase {
     Vecs<R> v = vecs(cs[1], nullptr, 0);
     v.f_out = k[0];
     launch_by_kind(KIND_RHS, v);
-    emit_commit_kernel<R><<<(unsigned)nblk_emit, kBlock, 0, stream>>>(emit_args());
+    launch_emit();
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(stream));
     begun = 1;
@@ -1384,6 +1428,7 @@ template <class R> struct Engine : EngineBase {
     HIP_TRY(hipEventCreate(&r0));
     HIP_TRY(hipEventCreate(&r1));
     std::vector<std::pair<hipEvent_t, hipEvent_t>> work = pairs_all;
+    launch_prepare();
     HIP_TRY(hipEventRecord(r0, stream));
     for (int a = 0; a < attempts; ++a) launch_attempt(&work);
     launch_finalize();

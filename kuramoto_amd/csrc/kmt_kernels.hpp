@@ -290,8 +290,10 @@ template <class R, int KIND> __device__ __forceinline__ RowOps<R, KIND> row_load
 // Row epilogue for oscillator i.  Returns the squared scaled error of
 // stage 7 (0 otherwise).  Stage combinations follow dp45.cu:34-69 with the
 // contraction acc = k1*a0; acc = fma(k_j, a_j, acc); y + h*acc -> fma(acc, h, y).
+// Stages 2..6 also hand back the (cos, sin) they write.
 template <class R, int KIND>
-__device__ __forceinline__ double row_finish(const Vecs<R> &a, long i, const RowOps<R, KIND> &o, R C, R S) {
+__device__ __forceinline__ double row_finish(const Vecs<R> &a, long i, const RowOps<R, KIND> &o, R C, R S,
+                                             R *c_out = nullptr, R *s_out = nullptr) {
   const R f = rhs_value<R>(o.om, a.c1, o.cs, o.sn, C, S);
   if constexpr (KIND == KIND_RHS) {
     a.f_out[i] = f;
@@ -315,6 +317,7 @@ __device__ __forceinline__ double row_finish(const Vecs<R> &a, long i, const Row
       rsincos<R>(yt, c, sn1);
       a.cs_out[i] = c;
       a.cs_out[a.ldv + i] = sn1;
+      if (c_out) { *c_out = c; *s_out = sn1; }
       return 0.0;
     } else {
       // embedded error, dp45.cu:79-84
@@ -747,138 +750,175 @@ __global__ __launch_bounds__(kBlock) void lowrank_expand_kernel(const R *X, int 
 // Low-rank coupling, one launch per RHS (K <= kLrMaxRank).
 //   G = w .* X^T (cos, sin) is formed in two halves: the launch that writes
 //   a stage vector also writes one partial sum of X^T (cos, sin) per
-//   workgroup (wave shuffles, then the wave sums in order); the next launch
-//   starts with every workgroup adding those partials in workgroup order
-//   (the same order in each, so all of them hold the same G), then computes
-//   C_i = sum_m X_im G_c[m], S_i likewise and the row epilogue of its stage.
-//   lowrank_gram_kernel writes the partials of a given vector (the first
-//   stage of an attempt, a stand-alone RHS).  No cross-workgroup
+//   workgroup (wave_reduce, then the wave sums in order); the next launch
+//   starts with every workgroup adding those partials (the same order in
+//   each, so all of them hold the same G), then computes C_i = sum_m X_im
+//   G_c[m], S_i likewise and the row epilogue of its stage.  The stage-2
+//   vector's partials come from lowrank_emit_kernel; lowrank_gram_kernel
+//   writes those of a given vector (a stand-alone RHS).  No cross-workgroup
 //   synchronisation inside a launch; partial buffers alternate between
 //   consecutive launches.
-// Rows are strided over a grid of at most kLrMaxBlocks workgroups.
+// The few MB it moves stay in the caches, so a launch is bound by latency:
+// one dependent round trip after another.  One row per thread up to
+// kLrMaxThreads x kLrMaxBlocks rows, in as few and as large workgroups as
+// still cover the CUs once (fewer partials for all of them to re-add: at
+// N=200000 241 workgroups of 832 threads, 19 KB of partials each, against
+// 512 of 256 threads that strode over 1.5 rows with 40 KB); the row's X
+// (from the transposed factor: coalesced), its epilogue operands and the
+// partials are all loaded before the first of them is needed; the rank is a
+// template argument up to 8 (no guards).  N=200000, K=5, FP32: 16.2 -> 7 us
+// per stage.
 // ---------------------------------------------------------------------
 constexpr int kLrMaxRank = 16;
 constexpr int kLrMaxBlocks = 512;
+constexpr int kLrMaxThreads = 1024;
+// larger ranks need the registers of 8 waves per CU (FP32 from 8, FP64 from 6
+// on 16 waves spill)
+constexpr int lr_max_threads(int real_bytes, int K) {
+  return K > (real_bytes == 8 ? 5 : 7) ? kLrMaxThreads / 2 : kLrMaxThreads;
+}
+template <class R, int KT> constexpr int kLrThreads = lr_max_threads(sizeof(R), KT);
+constexpr int lr_pow2(int n) { return n <= 1 ? 1 : 2 * lr_pow2((n + 1) / 2); }
 
-template <int KT>
-__device__ __forceinline__ void lr_write_partials(double (&acc)[2 * KT], int K, double *part) {
-  __shared__ double red[kBlock / kWave][2 * KT];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int nv = 2 * K;
+// A workgroup's sums of acc (2K values, interleaved c / s) -> part[q][block]
+template <class R, int KT>
+__device__ __forceinline__ void lr_write_partials(const double (&acc)[2 * KT], int K, double *part) {
+  constexpr int NV = lr_pow2(2 * KT);
+  __shared__ double red[kLrThreads<R, KT> / kWave][NV];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, nw = blockDim.x / kWave;
+  double v[NV];
 #pragma unroll
-  for (int q = 0; q < 2 * KT; ++q)
-    if (q < nv) {
-      const double t = wave_sum(acc[q]);
-      if (lane == 0) red[wave][q] = t;
-    }
+  for (int q = 0; q < NV; ++q) v[q] = q < 2 * KT ? acc[q < 2 * KT ? q : 0] : 0.0;
+  const double t = wave_reduce<double, NV>(v, lane);
+  red[wave][wave_slot<NV>(lane)] = t;
   __syncthreads();
-  if (threadIdx.x < nv) {
-    double t = red[0][threadIdx.x];
-#pragma unroll
-    for (int q = 1; q < kBlock / kWave; ++q) t += red[q][threadIdx.x];
-    part[(size_t)blockIdx.x * nv + threadIdx.x] = t;
+  if ((int)threadIdx.x < 2 * K) {
+    double s = red[0][threadIdx.x];
+    for (int q = 1; q < nw; ++q) s += red[q][threadIdx.x];
+    part[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
   }
 }
 
-// G (2K values, interleaved c/s) from nparts <= 2 kBlock partial vectors,
-// into g (LDS).  Thread t adds partials t and t + kBlock (all loads issued
-// at once), then the sums go through the wave shuffles and the wave order.
-static_assert(kLrMaxBlocks <= 2 * kBlock, "lr_reduce covers two partials per thread");
-template <class R, int KT>
-__device__ __forceinline__ void lr_reduce(const double *part, int nparts, int K, const R *w, double *g) {
-  __shared__ double red[kBlock / kWave][2 * KT];
+// G (2K values, interleaved c / s) from nparts partials of each, into g
+// (LDS): one wave per value, lane l adding partials l, l + 64, ...  lr_fetch
+// issues the first kLrPre loads of the wave's first value (before the
+// launch's state check; every buffer is readable then).
+constexpr int kLrPre = 4;
+__device__ __forceinline__ void lr_fetch(const double *part, int nparts, int K, double (&pre)[kLrPre]) {
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int nv = 2 * K;
-  const int b0 = threadIdx.x, b1 = threadIdx.x + kBlock;
-  double t0[2 * KT], t1[2 * KT];
 #pragma unroll
-  for (int q = 0; q < 2 * KT; ++q) {
-    t0[q] = (q < nv && b0 < nparts) ? part[(size_t)b0 * nv + q] : 0.0;
-    t1[q] = (q < nv && b1 < nparts) ? part[(size_t)b1 * nv + q] : 0.0;
+  for (int j = 0; j < kLrPre; ++j) {
+    const int b = lane + j * kWave;
+    pre[j] = wave < 2 * K && b < nparts ? part[(size_t)wave * nparts + b] : 0.0;
   }
-#pragma unroll
-  for (int q = 0; q < 2 * KT; ++q)
-    if (q < nv) {
-      const double t = wave_sum(t0[q] + t1[q]);
-      if (lane == 0) red[wave][q] = t;
-    }
-  __syncthreads();
-  if (threadIdx.x < 2 * KT) {
-    const int q = threadIdx.x;
+}
+template <class R>
+__device__ __forceinline__ void lr_reduce(const double *part, int nparts, int K, const R *w,
+                                          const double (&pre)[kLrPre], double *g) {
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, nw = blockDim.x / kWave;
+  for (int q = wave; q < 2 * K; q += nw) {
     double t = 0.0;
-    if (q < nv) {
-      t = red[0][q];
+    if (q == wave) {
 #pragma unroll
-      for (int r = 1; r < kBlock / kWave; ++r) t += red[r][q];
-      t *= (double)w[q >> 1];
+      for (int j = 0; j < kLrPre; ++j) t += pre[j];
     }
-    g[q] = t;
+#pragma unroll 4
+    for (int b = lane + (q == wave ? kLrPre * kWave : 0); b < nparts; b += kWave) t += part[(size_t)q * nparts + b];
+    t = wave_sum(t);
+    if (lane == 0) g[q] = t * (double)w[q >> 1];
   }
   __syncthreads();
 }
 
-template <class R, int KT>
-__global__ __launch_bounds__(kBlock) void lowrank_gram_kernel(const R *X, int K, long N, const R *cs, long ldv,
-                                                              double *part, const State<R> *st, int check_state) {
-  if (check_state && (!st->active || st->commit_pending)) return;
-  double acc[2 * KT];
+template <class R> struct LrArgs {
+  const R *XT;  // [K][ldv], zero past N
+  const R *w;   // [K]
+  int K;
+  const double *part_in;  // [2K][nparts]
+  int nparts;
+  double *part_out;       // [2K][gridDim.x]
+};
+
+template <class R, int KT, bool EXACT>
+__device__ __forceinline__ void lr_load_row(const LrArgs<R> &l, int K, long ldv, long i, R (&x)[KT]) {
 #pragma unroll
-  for (int q = 0; q < 2 * KT; ++q) acc[q] = 0.0;
-  for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < N; i += (long)gridDim.x * kBlock) {
-    const double c = cs[i], s = cs[ldv + i];
+  for (int m = 0; m < KT; ++m) x[m] = EXACT || m < K ? l.XT[m * ldv + i] : (R)0;
+}
+// acc += x (c, s) of one row; with a rank below KT the rows past it stay zero
+template <class R, int KT, bool EXACT>
+__device__ __forceinline__ void lr_accumulate(const R (&x)[KT], int K, R c, R s, double (&acc)[2 * KT]) {
 #pragma unroll
-    for (int m = 0; m < KT; ++m)
-      if (m < K) {
-        const double x = X[i * K + m];
-        acc[2 * m] = __builtin_fma(x, c, acc[2 * m]);
-        acc[2 * m + 1] = __builtin_fma(x, s, acc[2 * m + 1]);
-      }
-  }
-  lr_write_partials<KT>(acc, K, part);
+  for (int m = 0; m < KT; ++m)
+    if (EXACT || m < K) {
+      acc[2 * m] = __builtin_fma((double)x[m], (double)c, acc[2 * m]);
+      acc[2 * m + 1] = __builtin_fma((double)x[m], (double)s, acc[2 * m + 1]);
+    }
 }
 
-template <class R, int KIND, int KT, bool NEXT>
-__global__ __launch_bounds__(kBlock) void lowrank_stage_kernel(const R *X, int K, const double *part_in, int nparts,
-                                                               const R *w, Vecs<R> v, double *part_out) {
+template <class R, int KT, bool EXACT>
+__global__ __launch_bounds__((kLrThreads<R, KT>)) void lowrank_gram_kernel(const LrArgs<R> l, long N, const R *cs, long ldv) {
+  const int K = EXACT ? KT : l.K;
+  double acc[2 * KT] = {};
+  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) {
+    R x[KT];
+    lr_load_row<R, KT, EXACT>(l, K, ldv, i, x);
+    lr_accumulate<R, KT, EXACT>(x, K, cs[i], cs[ldv + i], acc);
+  }
+  lr_write_partials<R, KT>(acc, K, l.part_out);
+}
+
+template <class R, int KIND, int KT, bool EXACT>
+__global__ __launch_bounds__((kLrThreads<R, KT>)) void lowrank_stage_kernel(const LrArgs<R> l, const Vecs<R> v) {
+  constexpr bool NEXT = KIND >= 2 && KIND < 7;  // also the partials of the vector this stage writes
+  __shared__ double gs[2 * KT];
+  const int K = EXACT ? KT : l.K;
+  // everything the first row needs is in flight before the state check and
+  // the reduction of G (rows past N re-read row N - 1, never used)
+  const long stride = (long)gridDim.x * blockDim.x;
+  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  double pre[kLrPre];
+  lr_fetch(l.part_in, l.nparts, K, pre);
+  R x[KT];
+  const long i0 = i < v.N ? i : v.N - 1;
+  lr_load_row<R, KT, EXACT>(l, K, v.ldv, i0, x);
+  RowOps<R, KIND> ops = row_load<R, KIND>(v, i0);
+  asm volatile("" ::: "memory");
   if constexpr (KIND >= 2) {
     if (v.check_state && (!v.st->active || v.st->commit_pending)) return;
   }
-  __shared__ double errsq[kBlock];
-  __shared__ double gs[2 * KT];
-  lr_reduce<R, KT>(part_in, nparts, K, w, gs);
-  double g[2 * KT];
-#pragma unroll
-  for (int q = 0; q < 2 * KT; ++q) g[q] = gs[q];
-  double acc[2 * KT];
-#pragma unroll
-  for (int q = 0; q < 2 * KT; ++q) acc[q] = 0.0;
+  lr_reduce<R>(l.part_in, l.nparts, K, l.w, pre, gs);
+  double acc[2 * KT] = {};
   double sq = 0.0;
-  for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < v.N; i += (long)gridDim.x * kBlock) {
-    double x[KT];
+  while (i < v.N) {
+    asm volatile("" ::: "memory");  // G is re-read from LDS for every row: in registers it would cost 4K of them
     double C = 0, S = 0;
 #pragma unroll
     for (int m = 0; m < KT; ++m)
-      if (m < K) {
-        x[m] = X[i * K + m];
-        C = __builtin_fma(x[m], g[2 * m], C);
-        S = __builtin_fma(x[m], g[2 * m + 1], S);
+      if (EXACT || m < K) {
+        C = __builtin_fma((double)x[m], gs[2 * m], C);
+        S = __builtin_fma((double)x[m], gs[2 * m + 1], S);
       }
-    sq += row_epilogue<R, KIND>(v, i, (R)C, (R)S);
-    if constexpr (NEXT) {
-      const double c = v.cs_out[i], s = v.cs_out[v.ldv + i];
-#pragma unroll
-      for (int m = 0; m < KT; ++m)
-        if (m < K) {
-          acc[2 * m] = __builtin_fma(x[m], c, acc[2 * m]);
-          acc[2 * m + 1] = __builtin_fma(x[m], s, acc[2 * m + 1]);
-        }
+    R c = 0, s = 0;
+    sq += row_finish<R, KIND>(v, i, ops, (R)C, (R)S, &c, &s);
+    if constexpr (NEXT) lr_accumulate<R, KT, EXACT>(x, K, c, s, acc);
+    i += stride;
+    if (i < v.N) {
+      lr_load_row<R, KT, EXACT>(l, K, v.ldv, i, x);
+      ops = row_load<R, KIND>(v, i);
     }
   }
   if constexpr (KIND == 7) {
-    const double tot = block_sum(sq, errsq);
-    if (threadIdx.x == 0) v.err_part[blockIdx.x] = tot;
+    __shared__ double errsq[kLrThreads<R, KT> / kWave];
+    const double t = wave_sum(sq);
+    if (threadIdx.x % kWave == 0) errsq[threadIdx.x / kWave] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double tot = errsq[0];
+      for (int q = 1; q < (int)blockDim.x / kWave; ++q) tot += errsq[q];
+      v.err_part[blockIdx.x] = tot;
+    }
   }
-  if constexpr (NEXT) lr_write_partials<KT>(acc, K, part_out);
+  if constexpr (NEXT) lr_write_partials<R, KT>(acc, K, l.part_out);
 }
 
 // r = sqrt((X/N)^2 + (Y/N)^2) in the working precision (kuramoto.cu:220:
@@ -1158,6 +1198,84 @@ __global__ __launch_bounds__(kBlock) void emit_commit_kernel(const EmitArgs<R> a
     a.k[0][i] = k7;
     stage2_vector<R>(a, i, yn, k7, h);
   }
+}
+
+// emit_commit_kernel for the low-rank path, on its grid (threads stride over
+// the rows), with the partials of X^T (cos, sin) of the stage-2 vector it
+// writes.  Output rows four at a time: each wave's 8 sums by wave_reduce,
+// then the waves in order.
+template <class R, int KT, bool EXACT>
+__global__ __launch_bounds__((kLrThreads<R, KT>)) void lowrank_emit_kernel(const EmitArgs<R> a, const LrArgs<R> l) {
+  const State<R> *st = a.st;
+  const int mode = st->job_mode;
+  if (mode == JOB_NONE) return;
+  constexpr int ER = 4;
+  __shared__ double red[kLrThreads<R, KT> / kWave][2 * ER];
+  const int K = EXACT ? KT : l.K;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, nw = blockDim.x / kWave;
+  const long first = (long)blockIdx.x * blockDim.x + tid, stride = (long)gridDim.x * blockDim.x;
+  const R h = st->h;
+  const int n_emit = mode == JOB_STAGE2 ? 0 : st->job_n, slot0 = st->job_slot, lo = st->job_lo;
+  const R tl = st->t_last, hh = st->t - tl;
+  for (int q0 = 0; q0 < n_emit; q0 += ER) {
+    double v[2 * ER] = {};
+    for (long i = first; i < a.N; i += stride) {
+      R kv[7], Q[4];
+#pragma unroll
+      for (int j = 0; j < 7; ++j) kv[j] = a.k[j][i];
+      dense_coeffs<R>(kv, Q);
+      const R yl = a.y[i];
+#pragma unroll
+      for (int r = 0; r < ER; ++r) {
+        if (q0 + r >= n_emit) break;
+        const R val = dense_value<R>(Q, yl, hh, (a.t_eval[lo + q0 + r] - tl) / hh);
+        if (a.ring) a.ring[(size_t)(slot0 + q0 + r) * a.ldv + i] = val;
+        R c, s;
+        rsincos<R>(val, c, s);
+        v[2 * r] += (double)c;
+        v[2 * r + 1] += (double)s;
+      }
+    }
+    const double t = wave_reduce<double, 2 * ER>(v, lane);
+    red[wave][wave_slot<2 * ER>(lane)] = t;
+    __syncthreads();
+    if (tid < 2 * ER && q0 + tid / 2 < n_emit) {
+      double sum = red[0][tid];
+      for (int w = 1; w < nw; ++w) sum += red[w][tid];
+      a.ord_part[((size_t)(slot0 + q0 + tid / 2) * gridDim.x + blockIdx.x) * 2 + tid % 2] = sum;
+    }
+    __syncthreads();
+  }
+  if (mode == JOB_EMIT) return;
+  double acc[2 * KT] = {};
+  for (long i = first; i < a.N; i += stride) {
+    R x[KT];
+    lr_load_row<R, KT, EXACT>(l, K, a.ldv, i, x);
+    R y = a.y[i], k1 = a.k[0][i];
+    if (mode == JOB_COMMIT) {
+      // commit (dp45.cu:123-125, FSAL copy :160)
+      a.ylast[i] = y;
+      y = a.ynew[i];
+      k1 = a.k[6][i];
+      a.y[i] = y;
+      a.k[0][i] = k1;
+    }
+    const R yt = rfma<R>(k1 * (R)tab::A[0][0], h, y);
+    R c, s;
+    rsincos<R>(yt, c, s);
+    a.cs_out[i] = c;
+    a.cs_out[a.ldv + i] = s;
+    lr_accumulate<R, KT, EXACT>(x, K, c, s, acc);
+  }
+  lr_write_partials<R, KT>(acc, K, l.part_out);
+}
+
+// XT[m][i] = X[i][m] (XT cleared past N by its allocation)
+template <class R>
+__global__ __launch_bounds__(kBlock) void transpose_factor_kernel(const R *X, int K, long N, long ldv, R *XT) {
+  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
+  if (i < N)
+    for (int m = 0; m < K; ++m) XT[m * ldv + i] = X[i * K + m];
 }
 
 // ---------------------------------------------------------------------
