@@ -168,10 +168,62 @@ template <class R> __device__ __forceinline__ R rmax(R a, R b) {
   if constexpr (sizeof(R) == 4) return fmaxf(a, b); else return fmax(a, b);
 }
 
-template <class T> __device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
+// Exchanges between the lanes of a wave (all 64 active) in registers: the
+// swaps of the wave's halves and of its rows of 16, and DPP moves inside a
+// row.  Through LDS (a lane permute) every level of a sum waits for an LDS
+// round trip.
+template <class T, class F> __device__ __forceinline__ T lane_words(T v, F f) {
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(T, f(__builtin_bit_cast(uint32_t, v)));
+  } else {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    return __builtin_bit_cast(T, (uint64_t)f((uint32_t)(u >> 32)) << 32 | f((uint32_t)u));
+  }
+}
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_move(uint32_t w) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)w, CTRL, 0xF, 0xF, true);
+}
+// the value of lane ^ OFF (OFF = 8, 4, 2, 1)
+template <int OFF, class T> __device__ __forceinline__ T lane_xor(T v) {
+  return lane_words(v, [](uint32_t w) {
+    if constexpr (OFF == 8) return dpp_move<0x128>(w);                        // row rotated by 8
+    else if constexpr (OFF == 4) return dpp_move<0x1B>(dpp_move<0x141>(w));  // halves mirrored (^ 7), quads mirrored (^ 3)
+    else if constexpr (OFF == 2) return dpp_move<0x4E>(w);                    // quads 2 3 0 1
+    else return dpp_move<0xB1>(w);                                            // quads 1 0 3 2
+  });
+}
+// OFF = 32, 16: lanes with the bit clear get a[l] + a[l ^ OFF], the others
+// b[l ^ OFF] + b[l]
+template <int OFF, class T> __device__ __forceinline__ T lane_swap_sum(T a, T b) {
+  auto swap = [](uint32_t &x, uint32_t &y) {
+    if constexpr (OFF == 32) {
+      const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+      x = r[0], y = r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+      x = r[0], y = r[1];
+    }
+  };
+  if constexpr (sizeof(T) == 4) {
+    uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+    swap(x, y);
+    return __builtin_bit_cast(T, x) + __builtin_bit_cast(T, y);
+  } else {
+    const uint64_t u = __builtin_bit_cast(uint64_t, a), w = __builtin_bit_cast(uint64_t, b);
+    uint32_t xl = (uint32_t)u, yl = (uint32_t)w, xh = (uint32_t)(u >> 32), yh = (uint32_t)(w >> 32);
+    swap(xl, yl);
+    swap(xh, yh);
+    return __builtin_bit_cast(T, (uint64_t)xh << 32 | xl) + __builtin_bit_cast(T, (uint64_t)yh << 32 | yl);
+  }
+}
+// v + the partner's v at distance OFF
+template <int OFF, class T> __device__ __forceinline__ T lane_pair_sum(T v) {
+  if constexpr (OFF >= 16) return lane_swap_sum<OFF>(v, v);
+  else return v + lane_xor<OFF>(v);
+}
+template <class T, int OFF = kWave / 2> __device__ __forceinline__ T wave_sum(T v) {
+  if constexpr (OFF > 0) return wave_sum<T, OFF / 2>(lane_pair_sum<OFF>(v));
+  else return v;
 }
 
 // The NV values v[0..NV) of every lane, each summed over the wave in
@@ -190,15 +242,16 @@ template <class T, int HALF, int OFF, int NV> __device__ __forceinline__ T wave_
     const bool up = lane & OFF;
 #pragma unroll
     for (int k = 0; k < HALF; ++k) {
-      const T keep = up ? v[k + HALF] : v[k], send = up ? v[k] : v[k + HALF];
-      v[k] = keep + __shfl_xor(send, OFF, kWave);
+      if constexpr (OFF >= 16) {
+        v[k] = lane_swap_sum<OFF>(v[k], v[k + HALF]);
+      } else {
+        const T keep = up ? v[k + HALF] : v[k], send = up ? v[k] : v[k + HALF];
+        v[k] = keep + lane_xor<OFF>(send);
+      }
     }
     return wave_reduce_from<T, HALF / 2, OFF / 2>(v, lane);
   } else {
-    T s = v[0];
-#pragma unroll
-    for (int off = OFF; off > 0; off >>= 1) s += __shfl_xor(s, off, kWave);
-    return s;
+    return wave_sum<T, OFF>(v[0]);
   }
 }
 template <class T, int NV> __device__ __forceinline__ T wave_reduce(T (&v)[NV], int lane) {
