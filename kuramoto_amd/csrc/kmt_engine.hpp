@@ -117,6 +117,7 @@ template <class R> struct Engine : EngineBase {
   hipGraphExec_t g1 = nullptr, g8 = nullptr;
   bool graphs_valid = false;
   int tune_rows = 8, tune_nt = 1, tune_bal = 0, tune_ring = 0, tuned = 0;
+  int pinned = 0;  // variant chosen by the caller (kmt_select_variant, kmt_autotune)
   double tune_ms[12] = {0};
   int bal_grid = 0;  // workgroups of the balanced variant (one resident round)
   R t0_ = 0, h0_ = 0;
@@ -265,7 +266,7 @@ template <class R> struct Engine : EngineBase {
     tune_bal = (flags >> 1) & 1;
     tune_ring = (flags >> 2) & 1;
     bal_grid = 0;
-    tuned = 1;
+    tuned = pinned = 1;
     drop_graphs();
     return KMT_OK;
   }
@@ -380,7 +381,7 @@ template <class R> struct Engine : EngineBase {
     }
     A_bytes = bytes;
     storage = stg;
-    tuned = 0;
+    tuned = pinned = 0;
     bal_grid = 0;
     HIP_TRY(hipMemsetAsync(A, 0, bytes, stream));
     return KMT_OK;
@@ -1083,7 +1084,7 @@ template <class R> struct Engine : EngineBase {
     tune_bal = best_bal;
     tune_ring = best_ring;
     bal_grid = best_grid;
-    tuned = 1;
+    tuned = pinned = 1;
     drop_graphs();
     return KMT_OK;
   }
@@ -1142,6 +1143,51 @@ template <class R> struct Engine : EngineBase {
   // the order parameters of the last attempt's rows (earlier ones are
   // computed by the next attempt's control_kernel): before the host looks
   void launch_finalize() { finalize_kernel<R><<<1, kBlock, 0, stream>>>(st, ord_part, emit_blocks(), N, r_ring); }
+
+  // Small dense networks in the working precision: whole attempts in one
+  // workgroup, as far as its registers hold the matrix.  A caller's own
+  // choice of stage variant keeps the launched kernels.
+  bool small_path() const {
+    return !factored && A && storage == KMT_ADJ_NATIVE && !pinned && N <= kSmallMaxN<R>;
+  }
+  template <int G> void launch_small(const SmallArgs<R> &a, int n) {
+    if constexpr (G < kSmallMaxGroups<R>) {
+      if (N > (long)G * 8 * kSmallWaves) {
+        launch_small<G + 1>(a, n);
+        return;
+      }
+    }
+    small_attempts_kernel<R, G><<<1, kSmallThreads, 0, stream>>>(a, n);
+  }
+  // n attempts of the run
+  int launch_attempts(int n) {
+    if (small_path()) {
+      SmallArgs<R> a;
+      a.A = (const R *)A;
+      a.lda = lda;
+      a.N = N;
+      a.ldv = ldv;
+      a.omega = omega;
+      a.y = y;
+      a.ylast = ylast;
+      a.ynew = ynew;
+      for (int j = 0; j < 7; ++j) a.k[j] = k[j];
+      a.cs = cs[0];
+      a.c1 = c1;
+      a.st = st;
+      a.t_eval = t_eval;
+      a.times = times;
+      a.ring = keep_rows ? ring : nullptr;
+      a.r_ring = r_ring;
+      launch_small<1>(a, n);
+      HIP_TRY(hipGetLastError());
+      return KMT_OK;
+    }
+    if (!graphs_valid) KMT_TRY(build_graphs());
+    for (; n >= 8; n -= 8) HIP_TRY(hipGraphLaunch(g8, stream));
+    for (; n > 0; --n) HIP_TRY(hipGraphLaunch(g1, stream));
+    return KMT_OK;
+  }
 
   int build_graphs() {
     drop_graphs();
@@ -1292,11 +1338,7 @@ template <class R> struct Engine : EngineBase {
     if (max_attempts < 0) return fail(KMT_ERR_ARG, "max_attempts < 0");
     KMT_TRY(fetch_state());
     int n = std::min(max_attempts, shadow.times_cap - shadow.times_count);
-    if (shadow.active && n > 0) {
-      if (!graphs_valid) KMT_TRY(build_graphs());
-      for (; n >= 8; n -= 8) HIP_TRY(hipGraphLaunch(g8, stream));
-      for (; n > 0; --n) HIP_TRY(hipGraphLaunch(g1, stream));
-    }
+    if (shadow.active && n > 0) KMT_TRY(launch_attempts(n));
     KMT_TRY(fetch_state());
     fill_status(s);
     if (shadow.error) return fail(KMT_ERR_NUMERIC, "error norm is not finite at t=%g (h=%g): integration stopped", (double)shadow.t, (double)shadow.h);
@@ -1364,10 +1406,7 @@ template <class R> struct Engine : EngineBase {
     if (!begun) return fail(KMT_ERR_STATE, "kmt_step before kmt_begin");
     KMT_TRY(fetch_state());
     const long long before = shadow.accepted;
-    if (shadow.active && shadow.times_count < shadow.times_cap) {
-      if (!graphs_valid) KMT_TRY(build_graphs());
-      HIP_TRY(hipGraphLaunch(g1, stream));
-    }
+    if (shadow.active && shadow.times_count < shadow.times_cap) KMT_TRY(launch_attempts(1));
     KMT_TRY(fetch_state());
     if (acc) *acc = shadow.accepted > before ? 1 : 0;
     if (t) *t = (double)shadow.t;

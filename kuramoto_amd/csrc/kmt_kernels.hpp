@@ -24,6 +24,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace kmt {
 
 constexpr int kBlock = 256;  // threads per workgroup (4 waves of 64)
@@ -1004,44 +1006,34 @@ __device__ __forceinline__ void order_rows(int n, const double *part, int nblk, 
 }
 
 // ---------------------------------------------------------------------
-// Controller (dp45.cu:117-138): one workgroup, bound by the latency of its
-// chain of loads and of the norm's pow.  The state is read once at the start
-// (with the error partials in flight beside it), the decision is taken by
-// every lane of wave 0 in registers with the next 64 output times already
-// loaded, and written back once.
+// Controller (dp45.cu:117-138), in registers: every lane of one wave holds
+// the state S and updates it the same way.  err: sum of the squared scaled
+// errors (unused with a fixed step); te: output time e0 + lane, with e0 =
+// first pending or next output (NaN past the grid: never reached).  Lane 0
+// appends to the accepted-step log.
 // ---------------------------------------------------------------------
+template <class R> __device__ __forceinline__ int control_first_output(const State<R> &S) {
+  return S.commit_pending ? S.pend_lo : S.eval_i;
+}
 template <class R>
-__global__ __launch_bounds__(kBlock) void control_kernel(State<R> *st, const double *err_part, int nparts, long N,
-                                                         const R *t_eval, R *times, const double *ord_part, int nblk,
-                                                         R *r_ring) {
-  __shared__ double sh[kBlock];
-  double s = 0.0;
-#pragma unroll 8
-  for (int b = threadIdx.x; b < nparts; b += kBlock) s += err_part[b];
-  sh[threadIdx.x] = s;
-  const State<R> S = *st;
-  const int lane = threadIdx.x % kWave;
-  const int e0 = S.commit_pending ? S.pend_lo : S.eval_i;
-  R te = e0 + lane < S.n_eval ? t_eval[e0 + lane] : (R)NAN;  // NaN: never reached
-  if (S.fin_n > 0)  // the previous attempt's rows
-    order_rows<R>(S.fin_n, ord_part + (size_t)S.job_slot * nblk * 2, nblk, N, r_ring + S.job_slot);
-  __syncthreads();
-  if (threadIdx.x >= kWave) return;
-  int active = S.active, pending = S.commit_pending, lo = S.pend_lo, hi = S.pend_hi;
-  int mode = JOB_NONE, n_emit = 0;
-  R tn = S.t;
-  if (active && !pending) {
+__device__ __forceinline__ void control_decide(State<R> &S, double err, long N, const R *t_eval, R te, R *times,
+                                               int lane) {
+  S.job_mode = JOB_NONE;
+  S.job_n = S.fin_n = 0;
+  if (!S.active) return;
+  if (!S.commit_pending) {
     const R h = S.h;
-    int accept, error = 0;
+    int accept;
     R hnext = h;
-    double norm_d = S.norm;
+    S.attempts += 1;
+    S.rhs_evals += 6;
     if (S.fixed) {
       accept = 1;
     } else {
-      const R nrm = (R)sqrt(block_tree(sh));                     // {S,D}nrm2
+      const R nrm = (R)sqrt(err);                                // {S,D}nrm2
       const R norm = (R)((double)nrm / sqrt((double)N));        // dp45.cu:119
       R factor = (R)(0.9 * pow((double)norm, -0.2));            // dp45.cu:120
-      norm_d = (double)norm;
+      S.norm = (double)norm;
       if (norm < (R)1) {
         accept = 1;
         if (factor > (R)10) factor = (R)10;
@@ -1053,74 +1045,80 @@ __global__ __launch_bounds__(kBlock) void control_kernel(State<R> *st, const dou
           hnext = h * factor;
         }
         if (isnan((double)norm)) {  // the reference would loop forever here
-          error = 1;
-          active = 0;
+          S.error = 1;
+          S.active = 0;
         }
       }
     }
-    if (accept) {
-      tn = S.t + h;
-      // output times crossed by this step (kuramoto.cu:205-212): up to the
-      // first one not reached
-      lo = S.eval_i;
-      hi = lo;
-      for (;;) {
-        const unsigned long long miss = ~__ballot(tn >= te);
-        hi += miss ? __ffsll((long long)miss) - 1 : kWave;
-        if (miss) break;
-        te = hi + lane < S.n_eval ? t_eval[hi + lane] : (R)NAN;
-      }
-      pending = 1;
-    } else {
-      mode = active ? JOB_STAGE2 : JOB_NONE;
+    S.last_accept = accept;
+    S.h = hnext;
+    if (!accept) {
+      S.rejected += 1;
+      if (S.active) S.job_mode = JOB_STAGE2;
+      return;
     }
-    if (lane == 0) {
-      st->attempts = S.attempts + 1;
-      st->rhs_evals = S.rhs_evals + 6;
-      st->norm = norm_d;
-      st->last_accept = accept;
-      st->h = hnext;
-      if (accept) {
-        st->t_last = S.t;
-        st->t = tn;
-        st->accepted = S.accepted + 1;
-        if (S.times_count < S.times_cap) {
-          times[2 * S.times_count] = tn;
-          times[2 * S.times_count + 1] = hnext;
-          st->times_count = S.times_count + 1;
-        }
-      } else {
-        st->rejected = S.rejected + 1;
-        if (error) {
-          st->error = 1;
-          st->active = 0;
-        }
+    const R tn = S.t + h;
+    S.t_last = S.t;
+    S.t = tn;
+    S.accepted += 1;
+    if (S.times_count < S.times_cap) {
+      if (lane == 0) {
+        times[2 * S.times_count] = tn;
+        times[2 * S.times_count + 1] = hnext;
       }
+      S.times_count += 1;
     }
-  }
-  if (active && pending) {
-    const int room = S.ring_cap - S.ring_count;
-    n_emit = hi - lo < room ? hi - lo : room;
-    const bool all = n_emit == hi - lo;
-    mode = all ? JOB_COMMIT : JOB_EMIT;
-    if (lane == 0) {
-      st->job_lo = lo;
-      st->job_slot = S.ring_count;
-      st->ring_count = S.ring_count + n_emit;
-      st->pend_lo = lo + n_emit;
-      st->pend_hi = hi;
-      st->commit_pending = all ? 0 : 1;
-      if (all) {
-        st->eval_i = hi;
-        if (!(tn < S.t1)) st->active = 0;
-      }
+    // output times crossed by this step (kuramoto.cu:205-212): up to the
+    // first one not reached, 64 at a time
+    int hi = S.eval_i;
+    for (;;) {
+      const unsigned long long miss = ~__ballot(tn >= te);
+      hi += miss ? __ffsll((long long)miss) - 1 : kWave;
+      if (miss) break;
+      te = hi + lane < S.n_eval ? t_eval[hi + lane] : (R)NAN;
     }
+    S.pend_lo = S.eval_i;
+    S.pend_hi = hi;
+    S.commit_pending = 1;
   }
-  if (lane == 0) {
-    st->job_mode = mode;
-    st->job_n = n_emit;
-    st->fin_n = n_emit;
+  const int pend = S.pend_hi - S.pend_lo, room = S.ring_cap - S.ring_count;
+  S.job_n = S.fin_n = pend < room ? pend : room;
+  S.job_lo = S.pend_lo;
+  S.job_slot = S.ring_count;
+  S.job_mode = JOB_EMIT;
+  S.ring_count += S.job_n;
+  S.pend_lo += S.job_n;
+  if (S.job_n == pend) {
+    S.job_mode = JOB_COMMIT;
+    S.commit_pending = 0;
+    S.eval_i = S.pend_hi;
+    if (!(S.t < S.t1)) S.active = 0;
   }
+}
+
+// One workgroup, bound by the latency of its chain of loads and of the
+// norm's pow: the state is read once at the start, with the error partials
+// and then the next 64 output times in flight beside it, and written back
+// once.
+template <class R>
+__global__ __launch_bounds__(kBlock) void control_kernel(State<R> *st, const double *err_part, int nparts, long N,
+                                                         const R *t_eval, R *times, const double *ord_part, int nblk,
+                                                         R *r_ring) {
+  __shared__ double sh[kBlock];
+  double s = 0.0;
+#pragma unroll 8
+  for (int b = threadIdx.x; b < nparts; b += kBlock) s += err_part[b];
+  sh[threadIdx.x] = s;
+  State<R> S = *st;
+  const int lane = threadIdx.x % kWave;
+  const int e = control_first_output(S) + lane;
+  const R te = e < S.n_eval ? t_eval[e] : (R)NAN;
+  if (S.fin_n > 0)  // the previous attempt's rows
+    order_rows<R>(S.fin_n, ord_part + (size_t)S.job_slot * nblk * 2, nblk, N, r_ring + S.job_slot);
+  __syncthreads();
+  if (threadIdx.x >= kWave) return;
+  control_decide<R>(S, block_tree(sh), N, t_eval, te, times, lane);
+  if (lane == 0) *st = S;
 }
 
 // The order parameters control_kernel has not computed yet (after the last
@@ -1321,6 +1319,227 @@ __global__ __launch_bounds__((kLrThreads<R, KT>)) void lowrank_emit_kernel(const
     lr_accumulate<R, KT, EXACT>(x, K, c, s, acc);
   }
   lr_write_partials<R, KT>(acc, K, l.part_out);
+}
+
+// ---------------------------------------------------------------------
+// Small networks: whole attempts in one workgroup.
+// Between launches of 25 workgroups (N = 200) a stage is 3.6 us of latency:
+// a launch, the state check, one round trip for the rows, one for the
+// epilogue.  Up to N = 256 (FP32) or 128 (FP64) the whole matrix fits the
+// registers of one workgroup of 8 waves (G groups of 8 rows per wave, one
+// 16-byte piece per lane and row), so one workgroup runs attempt after
+// attempt in one launch: oscillator i's phase and k_j stay in thread i's
+// registers, the stage vectors in LDS, a stage is two barriers, and
+// kmt_advance needs no graph.  (Streaming a larger matrix into the one CU
+// from its L2 was slower than the launches: N=300 FP32 96 us per attempt
+// against 27.)  Sums, error partials, output rows and the controller follow
+// the launched kernels' order exactly (lane l's columns are those of thread l
+// of stage_ring_kernel, the only ones that see a column < 64 VEC; 8 rows per
+// error partial; 256 oscillators per order partial), so results are the same
+// bits.
+// ---------------------------------------------------------------------
+constexpr int kSmallThreads = 512;
+constexpr int kSmallWaves = kSmallThreads / kWave;
+template <class R> constexpr int kSmallMaxN = kWave * 16 / (int)sizeof(R);  // columns of one wave
+template <class R> constexpr int kSmallMaxGroups = kSmallMaxN<R> / (8 * kSmallWaves);
+
+template <class R> struct SmallArgs {
+  const R *A;
+  long lda, N, ldv;
+  const R *omega;
+  R *y, *ylast, *ynew;
+  R *k[7];
+  R *cs;  // the stage-2 vector between launches
+  R c1;
+  State<R> *st;
+  const R *t_eval;
+  R *times, *ring, *r_ring;
+};
+
+template <int I, int U, class F> __device__ __forceinline__ void small_unroll(F &&f) {
+  if constexpr (I < U) {
+    f(std::integral_constant<int, I>{});
+    small_unroll<I + 1, U>(f);
+  }
+}
+
+// The wave's rows: groups wave, wave + 8, ... of 8 rows, zero past the matrix
+template <class R, int G>
+__device__ __forceinline__ void small_load_rows(const SmallArgs<R> &a, u32x4 (&rows)[G][8]) {
+  const int wave = threadIdx.x / kWave, c = threadIdx.x % kWave * (16 / (int)sizeof(R));
+  small_unroll<0, G>([&](auto gi) {
+    constexpr int g = decltype(gi)::value;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const long row = (long)(g * kSmallWaves + wave) * 8 + r;
+      const bool in = c < a.lda && row < a.N;
+      const u32x4 raw = *reinterpret_cast<const u32x4 *>(a.A + (in ? row * a.lda + c : 0));
+      rows[g][r] = in ? raw : u32x4{0, 0, 0, 0};
+    }
+  });
+}
+
+// C, S of every row against the stage vector v (zero past N) -> sum
+template <class R, int G>
+__device__ __forceinline__ void small_row_sums(u32x4 (&rows)[G][8], const R (&v)[2][kSmallMaxN<R>],
+                                               double (&sum)[2][kSmallMaxN<R>]) {
+  constexpr int VEC = 16 / sizeof(R), ROWS = 8;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  R cv[VEC], sv[VEC];
+  load_reals<R, VEC>(v[0] + lane * VEC, cv);
+  load_reals<R, VEC>(v[1] + lane * VEC, sv);
+  small_unroll<0, G>([&](auto gi) {
+    constexpr int g = decltype(gi)::value;
+    double acc[2 * ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      // opaque: the conversions to double stay here (kept across stages they
+      // take twice the matrix's registers)
+      asm volatile("" : "+v"(rows[g][r]));
+      R m[VEC];
+      unpack<R>(rows[g][r], m);
+      acc[r] = acc[ROWS + r] = 0.0;
+#pragma unroll
+      for (int q = 0; q < VEC; ++q) {
+        acc[r] = __builtin_fma((double)m[q], (double)cv[q], acc[r]);
+        acc[ROWS + r] = __builtin_fma((double)m[q], (double)sv[q], acc[ROWS + r]);
+      }
+    }
+    const double t = wave_reduce<double, 2 * ROWS>(acc, lane);
+    const int slot = wave_slot<2 * ROWS>(lane);
+    sum[slot / ROWS][(g * kSmallWaves + wave) * ROWS + slot % ROWS] = t;
+    __builtin_amdgcn_sched_barrier(0);  // one group's sums in registers at a time
+  });
+}
+
+template <class R, int G>
+__global__ __launch_bounds__(kSmallThreads) void small_attempts_kernel(const SmallArgs<R> a, int attempts) {
+  constexpr int NMAX = kSmallMaxN<R>;
+  static_assert(NMAX <= kBlock && NMAX % 8 == 0, "one order partial; whole groups of rows");
+  __shared__ __align__(16) R v[2][2][NMAX];  // stage vectors (cos, sin), used alternately
+  __shared__ double sum[2][NMAX];            // C, S; squared errors
+  __shared__ double part[2][kBlock];         // error partials; (cos, sin) of an output row
+  __shared__ State<R> S;
+  u32x4 rows[G][8];
+  small_load_rows<R, G>(a, rows);
+  const int tid = threadIdx.x, lane = tid % kWave, N = (int)a.N;
+  const bool mine = tid < N;
+  R y = 0, yl = 0, yn = 0, om = 0, k[7] = {};
+  if (tid == 0) S = *a.st;
+  if (mine) {
+    y = a.y[tid], yl = a.ylast[tid], yn = a.ynew[tid], om = a.omega[tid];
+#pragma unroll
+    for (int j = 0; j < 7; ++j) k[j] = a.k[j][tid];
+  }
+  if (tid < NMAX) {
+    v[0][0][tid] = mine ? a.cs[tid] : (R)0;
+    v[0][1][tid] = mine ? a.cs[a.ldv + tid] : (R)0;
+    v[1][0][tid] = v[1][1][tid] = (R)0;
+  }
+  __syncthreads();
+  auto set_vector = [&](R yt, int buf) {
+    R c, s;
+    rsincos<R>(yt, c, s);
+    v[buf][0][tid] = c;
+    v[buf][1][tid] = s;
+  };
+  for (int at = 0; at < attempts; ++at) {
+    const int active = S.active, pending = S.commit_pending;
+    const R h = S.h;
+    __syncthreads();  // S is read by all before the controller rewrites it
+    if (!active) break;
+    if (!pending) {
+      // stages 2..7, one copy of the row sums: f of the vector in buffer
+      // s & 1 is k_s; the next vector goes to the other buffer
+      R err = 0;
+#pragma unroll 1
+      for (int s = 2; s <= 7; ++s) {
+        small_row_sums<R, G>(rows, v[s & 1], sum);
+        __syncthreads();
+        const int t = mine ? tid : 0;
+        const R f = rhs_value<R>(om, a.c1, v[s & 1][0][t], v[s & 1][1][t], (R)sum[0][t], (R)sum[1][t]);
+        R acc = 0;
+        small_unroll<2, 8>([&](auto stage) {
+          constexpr int S1 = decltype(stage)::value;
+          if (s != S1) return;
+          k[S1 - 1] = f;
+          acc = k[0] * (R)(S1 < 7 ? tab::A[S1 < 7 ? S1 - 1 : 0][0] : tab::E[0]);
+#pragma unroll
+          for (int j = 1; j < S1; ++j)
+            acc = rfma<R>(k[j], (R)(S1 < 7 ? tab::A[S1 < 7 ? S1 - 1 : 0][j] : tab::E[j]), acc);
+        });
+        if (s < 7) {
+          const R yt = rfma<R>(acc, h, y);
+          if (s == 6) yn = yt;
+          if (mine) set_vector(yt, (s + 1) & 1);
+        } else {
+          err = acc;
+        }
+        __syncthreads();
+      }
+      const R num = h * err;
+      const R den = rfma<R>(S.rtl, rmax<R>(rabs<R>(y), rabs<R>(yn)), S.atl);
+      const R e = num / den;
+      if (tid < NMAX) sum[0][tid] = mine ? (double)e * (double)e : 0.0;
+      __syncthreads();
+      if (tid < kBlock) {
+        double p = 0.0;
+        if (8 * tid < N) {
+          double q = 0.0;
+#pragma unroll
+          for (int r = 0; r < 8; ++r) q += sum[0][8 * tid + r];
+          p += q;
+        }
+        part[0][tid] = p;
+      }
+      __syncthreads();
+    }
+    if (tid < kWave) {
+      State<R> W = S;
+      const int o = control_first_output(W) + lane;
+      const R te = o < W.n_eval ? a.t_eval[o] : (R)NAN;
+      control_decide<R>(W, block_tree(part[0]), N, a.t_eval, te, a.times, lane);
+      W.fin_n = 0;  // the rows' order parameters follow here
+      if (lane == 0) S = W;
+    }
+    __syncthreads();
+    const int mode = S.job_mode, n_emit = S.job_n, slot0 = S.job_slot;
+    if (n_emit > 0) {
+      const R tl = S.t_last, hh = S.t - tl;
+      R Q[4];
+      dense_coeffs<R>(k, Q);
+      for (int q = 0; q < n_emit; ++q) {
+        R c = 0, s = 0;
+        if (mine) {
+          const R val = dense_value<R>(Q, y, hh, (a.t_eval[S.job_lo + q] - tl) / hh);
+          if (a.ring) a.ring[(size_t)(slot0 + q) * a.ldv + tid] = val;
+          rsincos<R>(val, c, s);
+        }
+        if (tid < kBlock) {
+          part[0][tid] = (double)c;
+          part[1][tid] = (double)s;
+        }
+        __syncthreads();
+        if (tid < kWave) {
+          const double X = block_tree(part[0]), Y = block_tree(part[1]);
+          if (lane == 0) a.r_ring[slot0 + q] = order_value<R>(X, Y, N);
+        }
+        __syncthreads();
+      }
+    }
+    if (mode == JOB_COMMIT) yl = y, y = yn, k[0] = k[6];
+    if (mine && (mode == JOB_COMMIT || mode == JOB_STAGE2)) set_vector(rfma<R>(k[0] * (R)tab::A[0][0], S.h, y), 0);
+    __syncthreads();
+    if (mode == JOB_EMIT) break;  // the ring is full: only the host can go on
+  }
+  if (tid == 0) *a.st = S;
+  if (mine) {
+    a.y[tid] = y, a.ylast[tid] = yl, a.ynew[tid] = yn;
+#pragma unroll
+    for (int j = 0; j < 7; ++j) a.k[j][tid] = k[j];
+    a.cs[tid] = v[0][0][tid];
+    a.cs[a.ldv + tid] = v[0][1][tid];
+  }
 }
 
 // XT[m][i] = X[i][m] (XT cleared past N by its allocation)
