@@ -273,18 +273,36 @@ __global__ __launch_bounds__(WAVES * kWave) void bgemm_kernel(const T *At, long 
       }
       __builtin_amdgcn_sched_group_barrier(0x008, F, 0);
     } else {
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
+      // Two or more bands: a set is the MT fragments of one (k-step, hi or
+      // lo); set s + 1 is read from LDS while the MT NT MFMAs of set s run.
+      // Reading each fragment right before its MFMAs left the LDS latency
+      // exposed once per set: 512-row workgroups, B = 64, N = 20000, split 6:
+      // 218 -> 199 us per product.
+      constexpr int SETS = 4 * NV;
+      u32x4 vb[2][MT];
+      auto frag = [&](int st, u32x4 (&dst)[MT]) {
+        const int ks = st / NV, q = st % NV;
         const int off = (lane % 32) * kLdsRow + 16 * ks + 8 * (lane / 32);
 #pragma unroll
-        for (int q = 0; q < NV; ++q)
+        for (int mt = 0; mt < MT; ++mt)
+          dst[mt] = *reinterpret_cast<const u32x4 *>(&sh[cur][q][mt * 32 * kLdsRow + off]);
+      };
+      frag(0, vb[0]);
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            const u32x4 vv = *reinterpret_cast<const u32x4 *>(&sh[cur][q][mt * 32 * kLdsRow + off]);
+      for (int st = 0; st < SETS; ++st) {
+        if (st + 1 < SETS) frag(st + 1, vb[(st + 1) & 1]);
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = mfma32<T>(vv, af[nt][ks], acc[mt][nt]);
-          }
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = mfma32<T>(vb[st & 1][mt], af[nt][st / NV], acc[mt][nt]);
       }
+      __builtin_amdgcn_sched_group_barrier(0x100, MT, 0);
+#pragma unroll
+      for (int i = 0; i < (SETS - 1) * MT; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, MT * NT, 0);
     }
   };
   // One chunk c held in A register set S (= (c - c0) mod (PF + 1)).  V^T is
@@ -855,6 +873,7 @@ struct kmt_batch {
   int begun = 0;
   // tiling (shared) / rows (grouped)
   int tile_var = 3, ksplit = 8, lo = 1;
+  int tiled = 0;  // tile chosen by the caller (kmt_batch_select_tile, kmt_batch_autotune)
   double tune_ms[96] = {0};  // (tile_var 0..5) x (split 1..16)
   hipGraphExec_t g1 = nullptr, g8 = nullptr;
   // proposer
@@ -1104,6 +1123,30 @@ struct kmt_batch {
     else if (mt_act == 3) gemm_mt<T, 3>();
     else gemm_mt<T, 4>();
   }
+  // Split-K without the caller's choice: the grid is (row blocks x split)
+  // workgroups of 256 rows, one per CU at a time, so a split costs whole
+  // rounds of its slab's chunks, and its partials are written here and read
+  // back by the epilogue.  Of the splits 1..16, the one with the smallest
+  // rounds (slab chunks t_chunk + 3 us) + partials at 5 TB/s, with t_chunk =
+  // 0.6 us + 0.34 us per 32 rows of hi + lo vectors (half without lo) as
+  // measured at B = 64 and 32, N = 20000.  There it picks 3 (240 workgroups,
+  // one round) instead of the former 8 (640, two and a half): 206 against 234
+  // us per product and 31 against 84 MB of partials per stage; at N = 8000 it
+  // keeps 8 (256 workgroups).  Chosen once per run for the whole batch, so
+  // that compacting the rows of finished instances does not change the sums.
+  void default_split() {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) cus = 1;
+    const long nkc = lda_shared / kKC, nrb = rows_shared / 256;
+    const double t_chunk = 0.6e-6 + 0.34e-6 * mt * (lo ? 1.0 : 0.5);
+    double best = 1e30;
+    for (int c = 1; c <= 16; ++c) {
+      const long slab = (nkc + c - 1) / c, rounds = (nrb * c + cus - 1) / cus;
+      const double t = rounds * (slab * t_chunk + 3e-6) + 2.0 * c * mpad * (double)ldn * sizeof(float) / 5e12;
+      if (t < best) best = t, ksplit = c;
+    }
+    tile_var = 3;
+  }
   void coupling(int check) {
     if (shared) {
       if (storage == KMT_ADJ_BF16) gemm_t<bf16_t>(); else gemm_t<f16_t>();
@@ -1252,6 +1295,7 @@ struct kmt_batch {
     drop_graphs();
     KMT_TRY(ensure_P());
     KMT_TRY(build_items());
+    if (shared && !tiled) default_split();
     if (t_eval) (void)hipFree(t_eval);
     if (ord_part) (void)hipFree(ord_part);
     if (r_ring) (void)hipFree(r_ring);
@@ -1495,6 +1539,7 @@ struct kmt_batch {
     (void)hipEventDestroy(e1);
     tile_var = bnt;
     ksplit = bks;
+    tiled = 1;
     drop_graphs();
     if (best_nt) *best_nt = bnt;
     if (best_split) *best_split = bks;
@@ -1507,6 +1552,7 @@ struct kmt_batch {
     if (split < 1 || split > 16) return kmt_fail(KMT_ERR_ARG, "split_k must be 1..16 (got %d)", split);
     tile_var = variant;
     ksplit = split;
+    tiled = 1;
     drop_graphs();
     return KMT_OK;
   }
