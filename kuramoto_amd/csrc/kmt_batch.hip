@@ -859,6 +859,11 @@ struct kmt_batch {
   float *r_ring = nullptr, *t_eval = nullptr;
   BInst *inst = nullptr;
   std::vector<BInst> host_inst;
+  // host_inst of a run equals the device's records (nothing launched since
+  // they were fetched) up to the rings' drained counts; inst_dirty: those are
+  // not written back yet.  r_host: the rings as of then (r_valid).
+  bool inst_fresh = false, inst_dirty = false, r_valid = false;
+  float *r_host = nullptr;  // pinned, B x ring_cap
   void *A = nullptr;
   size_t A_bytes = 0;
   std::vector<size_t> a_off;
@@ -899,6 +904,8 @@ struct kmt_batch {
                     inst, A, a_off_d, a_ld_d, items, mlp_w, log, log_count};
     for (void *p : ptrs)
       if (p) (void)hipFree(p);
+    if (r_host) (void)hipHostFree(r_host);
+    r_host = nullptr;
     if (stream) (void)hipStreamDestroy(stream);
     stream = nullptr;
   }
@@ -961,6 +968,7 @@ struct kmt_batch {
 
   int set_instance(int b, const float *omega, const float *theta, double c1, double t0, double h0) {
     if (b < 0 || b >= B) return kmt_fail(KMT_ERR_ARG, "instance %d out of range", b);
+    KMT_TRY(flush());  // host_inst is changed below
     HIP_TRY(hipMemcpyAsync(om + (size_t)b * ldn, omega, sizeof(float) * Nb[b], hipMemcpyHostToDevice, stream));
     HIP_TRY(hipMemcpyAsync(y + (size_t)b * ldn, theta, sizeof(float) * Nb[b], hipMemcpyHostToDevice, stream));
     HIP_TRY(hipStreamSynchronize(stream));
@@ -1006,6 +1014,7 @@ struct kmt_batch {
   // dense adjacency of instance b (or the shared one, b = -1) from a factor
   int set_factor(int b, const float *Xh, const float *wh, int K) {
     if (shared ? b != -1 : (b < 0 || b >= B)) return kmt_fail(KMT_ERR_ARG, "instance %d: use -1 for the shared adjacency", b);
+    KMT_TRY(flush());  // host_inst is changed below
     KMT_TRY(ensure_A());
     const long N = shared ? Nmax : Nb[b];
     double mx = 0;
@@ -1326,6 +1335,9 @@ struct kmt_batch {
       mpad_act = mpad;
       vhalf = B;
     }
+    inst_fresh = inst_dirty = r_valid = false;
+    if (r_host) HIP_TRY(hipHostFree(r_host));
+    r_host = nullptr;
     HIP_TRY(hipMemcpyAsync(inst, host_inst.data(), sizeof(BInst) * B, hipMemcpyHostToDevice, stream));
     // k1 = f(y) for every instance, then the first stage-2 vectors
     dim3 g2((unsigned)nblk, (unsigned)B);
@@ -1342,8 +1354,19 @@ struct kmt_batch {
   }
 
   int fetch() {
+    if (inst_fresh) return KMT_OK;
     HIP_TRY(hipMemcpyAsync(host_inst.data(), inst, sizeof(BInst) * B, hipMemcpyDeviceToHost, stream));
     HIP_TRY(hipStreamSynchronize(stream));
+    inst_fresh = begun;
+    return KMT_OK;
+  }
+  // before launches that change the records
+  int flush() {
+    if (inst_dirty) {
+      HIP_TRY(hipMemcpyAsync(inst, host_inst.data(), sizeof(BInst) * B, hipMemcpyHostToDevice, stream));
+      HIP_TRY(hipStreamSynchronize(stream));
+    }
+    inst_fresh = inst_dirty = r_valid = false;
     return KMT_OK;
   }
 
@@ -1375,6 +1398,7 @@ struct kmt_batch {
     for (const BInst &in : host_inst) any |= in.active;
     if (any && n > 0 && shared && compaction) KMT_TRY(compact());
     if (any && n > 0) {
+      KMT_TRY(flush());
       if (!g1) KMT_TRY(build_graphs());
       for (; n >= 8; n -= 8) HIP_TRY(hipGraphLaunch(g8, stream));
       for (; n > 0; --n) HIP_TRY(hipGraphLaunch(g1, stream));
@@ -1420,17 +1444,29 @@ struct kmt_batch {
     KMT_TRY(fetch());
     const int ready = host_inst[b].ring_count;
     const int n = std::min(std::max(max_n, 0), ready);
-    std::vector<float> buf(std::max(ready, 1));
-    if (ready) {
-      HIP_TRY(hipMemcpyAsync(buf.data(), r_ring + (size_t)b * ring_cap, sizeof(float) * ready, hipMemcpyDeviceToHost, stream));
-      HIP_TRY(hipStreamSynchronize(stream));
+    if (ready > 0) {
+      // the rings of all instances in one copy: drains of the others follow
+      if (!r_valid) {
+        if (!r_host) HIP_TRY(hipHostMalloc((void **)&r_host, sizeof(float) * (size_t)B * ring_cap, hipHostMallocDefault));
+        int most = 0;
+        for (const BInst &in : host_inst) most = std::max(most, in.ring_count);
+        HIP_TRY(hipMemcpy2DAsync(r_host, sizeof(float) * ring_cap, r_ring, sizeof(float) * ring_cap, sizeof(float) * most, B,
+                                 hipMemcpyDeviceToHost, stream));
+        HIP_TRY(hipStreamSynchronize(stream));
+        r_valid = true;
+      }
+      float *mine = r_host + (size_t)b * ring_cap;
+      for (int q = 0; q < n; ++q) r[q] = mine[q];
+      if (n > 0) {
+        if (n < ready) {  // keep the unread values at the front
+          std::memmove(mine, mine + n, sizeof(float) * (ready - n));
+          HIP_TRY(hipMemcpyAsync(r_ring + (size_t)b * ring_cap, mine, sizeof(float) * (ready - n), hipMemcpyHostToDevice, stream));
+          HIP_TRY(hipStreamSynchronize(stream));
+        }
+        host_inst[b].ring_count = ready - n;
+        inst_dirty = true;
+      }
     }
-    for (int q = 0; q < n; ++q) r[q] = buf[q];
-    if (n < ready) HIP_TRY(hipMemcpyAsync(r_ring + (size_t)b * ring_cap, buf.data() + n, sizeof(float) * (ready - n), hipMemcpyHostToDevice, stream));
-    const int left = ready - n;
-    HIP_TRY(hipMemcpyAsync(&inst[b].ring_count, &left, sizeof(int), hipMemcpyHostToDevice, stream));
-    HIP_TRY(hipStreamSynchronize(stream));
-    host_inst[b].ring_count = left;
     if (nout) *nout = n;
     return KMT_OK;
   }
@@ -1453,6 +1489,7 @@ struct kmt_batch {
 
   int time_attempts(int attempts, double *region_ms, double *coupling_ms, kmt_batch_status *s) {
     if (!begun) return kmt_fail(KMT_ERR_STATE, "kmt_batch_time_attempts before kmt_batch_begin");
+    KMT_TRY(flush());
     std::vector<std::pair<hipEvent_t, hipEvent_t>> all(6 * attempts);
     for (auto &p : all) {
       HIP_TRY(hipEventCreate(&p.first));

@@ -76,7 +76,17 @@ template <class R> struct Engine : EngineBase {
   double *ord_scr = nullptr;  // stand-alone order parameter partials + result
   State<R> *st = nullptr;
   State<R> *st_host = nullptr;  // pinned
+  // Host copy of the device state.  fresh: equal to it up to the host's own
+  // drains (nothing launched since it was fetched), so reading entry points
+  // need no round trip; dirty: drains not yet sent, written back before the
+  // next launch that uses the state.
   State<R> shadow{};
+  bool fresh = false, dirty = false;
+  // pinned staging of row drains (two halves, grown to at most kStageMax each)
+  static constexpr size_t kStageMax = (size_t)1 << 20;
+  char *stage_buf = nullptr;
+  size_t stage_half = 0;
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};
 
   // adjacency
   int storage = -1;  // KMT_ADJ_*
@@ -139,6 +149,9 @@ template <class R> struct Engine : EngineBase {
     if (sym_prow) (void)hipFree(sym_prow);
     if (sym_pcol) (void)hipFree(sym_pcol);
     if (st_host) (void)hipHostFree(st_host);
+    if (stage_buf) (void)hipHostFree(stage_buf);
+    for (hipEvent_t e : stage_ev)
+      if (e) (void)hipEventDestroy(e);
     if (A) (void)hipFree(A);
     if (stream) (void)hipStreamDestroy(stream);
     y = ylast = ynew = omega = kbuf = nullptr;
@@ -292,9 +305,11 @@ template <class R> struct Engine : EngineBase {
   }
 
   int fetch_state() {
+    if (fresh) return KMT_OK;
     HIP_TRY(hipMemcpyAsync(st_host, st, sizeof(State<R>), hipMemcpyDeviceToHost, stream));
     HIP_TRY(hipStreamSynchronize(stream));
     shadow = *st_host;
+    fresh = true;
     return KMT_OK;
   }
 
@@ -302,6 +317,65 @@ template <class R> struct Engine : EngineBase {
     *st_host = shadow;
     HIP_TRY(hipMemcpyAsync(st, st_host, sizeof(State<R>), hipMemcpyHostToDevice, stream));
     HIP_TRY(hipStreamSynchronize(stream));
+    fresh = true;
+    dirty = false;
+    return KMT_OK;
+  }
+  // before launches that change the state (fetch_state waits for them before
+  // st_host is used again)
+  int flush_state() {
+    if (dirty) {
+      *st_host = shadow;
+      HIP_TRY(hipMemcpyAsync(st, st_host, sizeof(State<R>), hipMemcpyHostToDevice, stream));
+      dirty = false;
+    }
+    fresh = false;
+    return KMT_OK;
+  }
+
+  // `rows` rows of `width` bytes to host memory.  Pinned memory is written
+  // directly.  A pitched copy into pageable memory took 0.5 ms for six rows of
+  // 20 KB and 2 ms for 190 of 40 KB; here whole stretches of the source go to
+  // a pinned half buffer while the other half is spread over the caller's rows.
+  int drain_rows(void *dst, const void *src, size_t pitch, size_t width, size_t rows) {
+    hipPointerAttribute_t at{};
+    const hipError_t known = hipPointerGetAttributes(&at, dst);
+    if (known == hipSuccess && at.type == hipMemoryTypeHost) {
+      HIP_TRY(hipMemcpy2DAsync(dst, width, src, pitch, width, rows, hipMemcpyDeviceToHost, stream));
+      return KMT_OK;
+    }
+    if (known != hipSuccess) (void)hipGetLastError();  // an address the runtime does not know is no error here
+    const size_t total = (rows - 1) * pitch + width;
+    const size_t half = std::min(kStageMax, std::max<size_t>((total + 1) / 2, 4096));
+    if (stage_half < half) {
+      if (stage_buf) HIP_TRY(hipHostFree(stage_buf));
+      stage_buf = nullptr;
+      stage_half = 0;
+      HIP_TRY(hipHostMalloc((void **)&stage_buf, 2 * half, hipHostMallocDefault));
+      stage_half = half;
+      for (hipEvent_t &e : stage_ev)
+        if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+    const size_t chunks = (total + stage_half - 1) / stage_half;
+    auto start = [&](size_t c) -> int {
+      const size_t o = c * stage_half, n = std::min(stage_half, total - o);
+      HIP_TRY(hipMemcpyAsync(stage_buf + (c & 1) * stage_half, (const char *)src + o, n, hipMemcpyDeviceToHost, stream));
+      HIP_TRY(hipEventRecord(stage_ev[c & 1], stream));
+      return KMT_OK;
+    };
+    KMT_TRY(start(0));
+    for (size_t c = 0; c < chunks; ++c) {
+      if (c + 1 < chunks) KMT_TRY(start(c + 1));
+      HIP_TRY(hipEventSynchronize(stage_ev[c & 1]));
+      const size_t o = c * stage_half, end = o + std::min(stage_half, total - o);
+      for (size_t q = o; q < end;) {  // the pieces of rows in [o, end)
+        const size_t row = q / pitch, col = q % pitch, next = std::min(end, (row + 1) * pitch);
+        if (col < width)
+          std::memcpy((char *)dst + row * width + col, stage_buf + (c & 1) * stage_half + (q - o),
+                      std::min(next - q, width - col));
+        q = next;
+      }
+    }
     return KMT_OK;
   }
 
@@ -1338,7 +1412,10 @@ template <class R> struct Engine : EngineBase {
     if (max_attempts < 0) return fail(KMT_ERR_ARG, "max_attempts < 0");
     KMT_TRY(fetch_state());
     int n = std::min(max_attempts, shadow.times_cap - shadow.times_count);
-    if (shadow.active && n > 0) KMT_TRY(launch_attempts(n));
+    if (shadow.active && n > 0) {
+      KMT_TRY(flush_state());
+      KMT_TRY(launch_attempts(n));
+    }
     KMT_TRY(fetch_state());
     fill_status(s);
     if (shadow.error) return fail(KMT_ERR_NUMERIC, "error norm is not finite at t=%g (h=%g): integration stopped", (double)shadow.t, (double)shadow.h);
@@ -1356,8 +1433,11 @@ template <class R> struct Engine : EngineBase {
     const int n = std::min(std::max(max_rows, 0), ready);
     if ((rows || cpl) && n > 0 && !keep_rows) return fail(KMT_ERR_STATE, "rows were not kept (kmt_begin keep_rows=0)");
     if (cpl && n > 0 && !coupling_ready()) return fail(KMT_ERR_STATE, "no adjacency for the couplings");
-    if (rows && n > 0)
-      HIP_TRY(hipMemcpy2DAsync(rows, sizeof(R) * N, ring, sizeof(R) * ldv, sizeof(R) * N, n, hipMemcpyDeviceToHost, stream));
+    if (ready == 0) {
+      if (nout) *nout = 0;
+      return KMT_OK;
+    }
+    if (rows && n > 0) KMT_TRY(drain_rows(rows, ring, sizeof(R) * ldv, sizeof(R) * N, n));
     for (int q = 0; cpl && q < n; ++q) {
       sincos_kernel<R><<<(unsigned)((N + kBlock - 1) / kBlock), kBlock, 0, stream>>>(ring + (size_t)q * ldv, N, ldv, cs_scr);
       Vecs<R> v = vecs(cs_scr, nullptr, 0);
@@ -1374,7 +1454,7 @@ template <class R> struct Engine : EngineBase {
       HIP_TRY(hipMemcpyAsync(r_ring + (q - n), r_ring + q, sizeof(R), hipMemcpyDeviceToDevice, stream));
     }
     shadow.ring_count = ready - n;
-    HIP_TRY(hipMemcpyAsync(&st->ring_count, &shadow.ring_count, sizeof(int), hipMemcpyHostToDevice, stream));
+    dirty = true;
     HIP_TRY(hipStreamSynchronize(stream));
     if (nout) *nout = n;
     return KMT_OK;
@@ -1385,19 +1465,21 @@ template <class R> struct Engine : EngineBase {
     KMT_TRY(fetch_state());
     const int ready = shadow.times_count;
     const int n = std::min(std::max(max_n, 0), ready);
-    std::vector<R> buf(2 * std::max(ready, 1));
     if (ready > 0) {
+      std::vector<R> buf(2 * ready);
       HIP_TRY(hipMemcpyAsync(buf.data(), times, sizeof(R) * 2 * ready, hipMemcpyDeviceToHost, stream));
       HIP_TRY(hipStreamSynchronize(stream));
+      for (int q = 0; q < n; ++q) {
+        if (tv) ((R *)tv)[q] = buf[2 * q];
+        if (hv) ((R *)hv)[q] = buf[2 * q + 1];
+      }
+      if (n > 0 && n < ready) {
+        HIP_TRY(hipMemcpyAsync(times, buf.data() + 2 * n, sizeof(R) * 2 * (ready - n), hipMemcpyHostToDevice, stream));
+        HIP_TRY(hipStreamSynchronize(stream));
+      }
+      shadow.times_count = ready - n;
+      dirty = true;
     }
-    for (int q = 0; q < n; ++q) {
-      if (tv) ((R *)tv)[q] = buf[2 * q];
-      if (hv) ((R *)hv)[q] = buf[2 * q + 1];
-    }
-    if (n < ready) HIP_TRY(hipMemcpyAsync(times, buf.data() + 2 * n, sizeof(R) * 2 * (ready - n), hipMemcpyHostToDevice, stream));
-    shadow.times_count = ready - n;
-    HIP_TRY(hipMemcpyAsync(&st->times_count, &shadow.times_count, sizeof(int), hipMemcpyHostToDevice, stream));
-    HIP_TRY(hipStreamSynchronize(stream));
     if (nout) *nout = n;
     return KMT_OK;
   }
@@ -1406,7 +1488,10 @@ template <class R> struct Engine : EngineBase {
     if (!begun) return fail(KMT_ERR_STATE, "kmt_step before kmt_begin");
     KMT_TRY(fetch_state());
     const long long before = shadow.accepted;
-    if (shadow.active && shadow.times_count < shadow.times_cap) KMT_TRY(launch_attempts(1));
+    if (shadow.active && shadow.times_count < shadow.times_cap) {
+      KMT_TRY(flush_state());
+      KMT_TRY(launch_attempts(1));
+    }
     KMT_TRY(fetch_state());
     if (acc) *acc = shadow.accepted > before ? 1 : 0;
     if (t) *t = (double)shadow.t;
@@ -1467,6 +1552,7 @@ template <class R> struct Engine : EngineBase {
     HIP_TRY(hipEventCreate(&r0));
     HIP_TRY(hipEventCreate(&r1));
     std::vector<std::pair<hipEvent_t, hipEvent_t>> work = pairs_all;
+    KMT_TRY(flush_state());
     launch_prepare();
     HIP_TRY(hipEventRecord(r0, stream));
     for (int a = 0; a < attempts; ++a) launch_attempt(&work);
