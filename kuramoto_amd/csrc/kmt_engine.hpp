@@ -108,8 +108,10 @@ template <class R> struct Engine : EngineBase {
   // the B fragments of the digits and the int32 partial sums
   int sign = 0;
   struct SignPass {
-    long ldp = 0, nsb = 0, npairs = 0, pairs_per = 1;  // nsb = 2 npairs super-blocks of 512
-    int nsplit = 1;
+    long ldp = 0, nsb = 0, npairs = 0;  // nsb = 2 npairs super-blocks of 512
+    long units = 1;       // row groups of 256 x pairs
+    int wgs = 1;          // workgroups that share the units
+    int nsplit = 1;       // most workgroups of one row group: slots of part
     uint32_t *tiles = nullptr;
     uint8_t *bfrag = nullptr;
     int32_t *part = nullptr;
@@ -627,38 +629,30 @@ template <class R> struct Engine : EngineBase {
 
   // 16-row tiles per wave of the int8 passes
   static constexpr int kSignNT = 4;
-  // Shape of a pass with `rows` output rows (+ the ones row) over kdim:
-  // workgroups of 4 row groups of 16 kSignNT rows x splits of the 1024-wide
-  // super-block pairs, at least 2 pairs per split.  The split count keeps
-  // the waves within two rounds of the `resident` waves the device holds at
-  // once and, among those counts, fills the last round best: a wave count
-  // just past a whole round leaves most of the GPU idle behind a few waves.
-  // N = K = 10^5 on 256 CUs at 3 workgroups per CU (3072 resident waves):
-  // 3 splits = 4692 waves = 1.53 rounds, 0.514-0.532 ms per RHS; 2 splits
-  // (1.02 rounds) 0.577, 4 (2.04) 0.551, 5 (2.55) 0.535, 6 (3.05) 0.563,
-  // 7 (3.56) 0.551; fewer splits also write and re-read fewer partials.
+  // Shape of a pass with `rows` output rows (+ the ones row) over kdim: the
+  // (row group, pair) units in equal stretches over the workgroups that the
+  // device holds at once, at least 2 pairs each (a pass of N = K = 10^4 is
+  // 400 units, 200 workgroups: latency-bound either way, and fewer partials).
   static constexpr long kSignRowsPerBlock = 16 * kSignNT * (kBlock / kWave);
   static SignPass sign_pass_shape(long rows, long kdim, long resident) {
     SignPass p;
     p.ldp = (rows + 1 + kSignRowsPerBlock - 1) / kSignRowsPerBlock * kSignRowsPerBlock;
-    const long rg = p.ldp / (16 * kSignNT);
+    const long groups = p.ldp / kSignRowsPerBlock;
     p.npairs = std::max<long>(1, (kdim + 2 * kSignSB - 1) / (2 * kSignSB));
     p.nsb = 2 * p.npairs;
-    const long spmax = std::min<long>(std::max<long>(1, 2 * resident / rg), std::max<long>(1, p.npairs / 2));
-    long sp = 1;
-    double best = -1.0;
-    for (long c = 1; c <= spmax; ++c) {
-      const long w = rg * c, rounds = (w + resident - 1) / resident;
-      const double fill = (double)w / (double)(rounds * resident);
-      if (fill > best) best = fill, sp = c;
-    }
-    p.pairs_per = (p.npairs + sp - 1) / sp;
-    p.nsplit = (int)((p.npairs + p.pairs_per - 1) / p.pairs_per);
+    p.units = groups * p.npairs;
+    p.wgs = (int)std::min(resident, std::max<long>(1, p.units / 2));
+    p.nsplit = 1;
+    for (long g = 0; g < groups; ++g)
+      p.nsplit = std::max(p.nsplit, (int)(sign_unit_owner((g + 1) * p.npairs - 1, p.units, p.wgs) -
+                                          sign_unit_owner(g * p.npairs, p.units, p.wgs) + 1));
     return p;
   }
   int alloc_sign_pass(SignPass &p, long kdim) {
     HIP_TRY(hipMalloc((void **)&p.bfrag, (size_t)p.nsb * 8 * kWave * 16));
+    // slots that a row group does not reach stay as cleared here
     HIP_TRY(hipMalloc((void **)&p.part, sizeof(int32_t) * 16 * (size_t)p.nsplit * p.ldp));
+    HIP_TRY(hipMemsetAsync(p.part, 0, sizeof(int32_t) * 16 * (size_t)p.nsplit * p.ldp, stream));
     std::vector<uint32_t> ones((size_t)16 * p.nsb, 0u);
     for (long q = 0; q < (long)ones.size(); ++q)
       ones[q] = 32 * (q + 1) <= kdim ? 0xFFFFFFFFu : (32 * q < kdim ? (1u << (kdim - 32 * q)) - 1u : 0u);
@@ -693,7 +687,7 @@ template <class R> struct Engine : EngineBase {
         per_cu < 1)
       per_cu = 1;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) cus = 1;
-    const long resident = (long)per_cu * cus * (kBlock / kWave);
+    const long resident = (long)per_cu * cus;
     s_pass[0] = sign_pass_shape(K, N, resident);
     s_pass[1] = sign_pass_shape(N, K, resident);
     SignPass &p1 = s_pass[0], &p2 = s_pass[1];
@@ -711,7 +705,7 @@ template <class R> struct Engine : EngineBase {
     // zero rows (and words past each row's k range) stay as cleared here
     HIP_TRY(hipMemsetAsync(p1.tiles, 0, sizeof(uint32_t) * tw1, stream));
     HIP_TRY(hipMemsetAsync(p2.tiles, 0, sizeof(uint32_t) * tw2, stream));
-    const size_t words = (size_t)((N + 63) / 64) * p2.npairs * 2048;
+    const size_t words = (size_t)((N + 255) / 256) * p2.npairs * 8192;
     gen_sign_bits_kernel<<<(unsigned)((words + kBlock - 1) / kBlock), kBlock, 0, stream>>>(p2.tiles, N, K, p2.npairs,
                                                                                           seed);
     HIP_TRY(hipGetLastError());
@@ -1021,17 +1015,14 @@ template <class R> struct Engine : EngineBase {
     const SignPass &p1 = s_pass[0], &p2 = s_pass[1];
     if (K > 0) {
       const long n_pad = p1.nsb * kSignSB, k_pad = p2.nsb * kSignSB;
-      const long b1 = (p1.ldp / kSignRowsPerBlock) * p1.nsplit, b2 = (p2.ldp / kSignRowsPerBlock) * p2.nsplit;
       sign_limbs_kernel<R><<<(unsigned)((n_pad + kBlock - 1) / kBlock), kBlock, 0, stream>>>(
           v.cs_in, v.cs_in + ldv, N, n_pad, p1.bfrag, st, chk);
-      sign_mfma_kernel<R, kSignNT><<<(unsigned)b1, kBlock, 0, stream>>>(
-          (const u32x4 *)p1.tiles, (const u32x4 *)p1.bfrag, p1.npairs, p1.pairs_per, p1.nsplit,
-          p1.part, p1.ldp, st, chk);
+      sign_mfma_kernel<R, kSignNT><<<(unsigned)p1.wgs, kBlock, 0, stream>>>(
+          (const u32x4 *)p1.tiles, (const u32x4 *)p1.bfrag, (int)p1.npairs, p1.units, p1.part, p1.ldp, st, chk);
       sign_gram_kernel<R><<<(unsigned)((k_pad + kBlock - 1) / kBlock), kBlock, 0, stream>>>(
           p1.part, p1.nsplit, p1.ldp, w, K, k_pad, p2.bfrag, st, chk);
-      sign_mfma_kernel<R, kSignNT><<<(unsigned)b2, kBlock, 0, stream>>>(
-          (const u32x4 *)p2.tiles, (const u32x4 *)p2.bfrag, p2.npairs, p2.pairs_per, p2.nsplit, p2.part,
-          p2.ldp, st, chk);
+      sign_mfma_kernel<R, kSignNT><<<(unsigned)p2.wgs, kBlock, 0, stream>>>(
+          (const u32x4 *)p2.tiles, (const u32x4 *)p2.bfrag, (int)p2.npairs, p2.units, p2.part, p2.ldp, st, chk);
     }
     sign_stage_kernel<R, KIND><<<(unsigned)((N + kBlock - 1) / kBlock), kBlock, 0, stream>>>(
         p2.part, K > 0 ? p2.nsplit : 0, p2.ldp, v);

@@ -65,18 +65,19 @@ __device__ __forceinline__ uint32_t sign_stream_word(uint64_t W, uint32_t seed) 
   return sel == 0 ? x[0] : sel == 1 ? x[1] : sel == 2 ? x[2] : x[3];
 }
 
-// Tile order of a pass's bits: rows in groups of 64 (one wave's four 16-row
-// MFMA tiles), words in pairs of 32 (1024 k, two super-blocks); the group's
-// 64 rows x 32 words of pair P are 8 KB of consecutive memory, in the order
-// one wave loads them: load (t, s) of lane (g, rl) is the 16 bytes of row
-// 16 t + rl, words 32 P + 8 g + 4 s .. + 3, at 16-byte slot
-// (2 t + s) 64 + 16 g + rl.  A wave thus streams one contiguous run as P
-// advances (row-major bits gave each lane's row 128 bytes every pair, rows
-// 12.5 KB apart at N = 10^5, and HBM served that at about half its rate).
+// Tile order of a pass's bits: rows in groups of 256 (a workgroup's four waves
+// of four 16-row MFMA tiles), words in pairs of 32 (1024 k, two super-blocks);
+// the group's 256 rows x 32 words of pair P are 32 KB of consecutive memory,
+// 8 KB per wave in the order it loads them: load (t, s) of lane (g, rl) is the
+// 16 bytes of row 16 t + rl of the wave, words 32 P + 8 g + 4 s .. + 3, at
+// 16-byte slot (2 t + s) 64 + 16 g + rl.  A workgroup thus streams one
+// contiguous run as P advances (row-major bits gave each lane's row 128 bytes
+// every pair, rows 12.5 KB apart at N = 10^5, and HBM served that at about
+// half its rate; 8 KB runs per wave, 800 KB apart, were 2.5% slower).
 __host__ __device__ __forceinline__ size_t sign_tile_word(long r, long q, long npairs) {
-  const long rg = r >> 6, t = (r >> 4) & 3, rl = r & 15;
+  const long rgb = r >> 8, w = (r >> 6) & 3, t = (r >> 4) & 3, rl = r & 15;
   const long P = q >> 5, g = (q >> 3) & 3, s = (q >> 2) & 1, e = q & 3;
-  return ((((size_t)rg * npairs + P) * 8 + (2 * t + s)) * 64 + (16 * g + rl)) * 4 + e;
+  return (((((size_t)rgb * npairs + P) * 4 + w) * 8 + (2 * t + s)) * 64 + (16 * g + rl)) * 4 + e;
 }
 
 // Row n of the pass-2 tiles, word q: signs of m = 32 q .. 32 q + 31 (m < K):
@@ -86,9 +87,9 @@ __host__ __device__ __forceinline__ size_t sign_tile_word(long r, long q, long n
 [[maybe_unused]] static __global__ __launch_bounds__(kBlock) void gen_sign_bits_kernel(uint32_t *tiles, long N, long K,
                                                                                       long npairs, uint32_t seed) {
   const long o = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (o >= (N + 63) / 64 * npairs * 2048) return;
-  const long piece = o >> 2, lane = piece & 63, ts = (piece >> 6) & 7, tile = piece >> 9;
-  const long n = 64 * (tile / npairs) + 16 * (ts >> 1) + (lane & 15);
+  if (o >= (N + 255) / 256 * npairs * 8192) return;
+  const long piece = o >> 2, lane = piece & 63, ts = (piece >> 6) & 7, w = (piece >> 9) & 3, tile = piece >> 11;
+  const long n = 256 * (tile / npairs) + 64 * w + 16 * (ts >> 1) + (lane & 15);
   const long q = 32 * (tile % npairs) + 8 * (lane >> 4) + 4 * (ts & 1) + (o & 3);
   if (n >= N) return;  // the ones row and zero rows are written separately
   uint32_t word = 0;
@@ -154,19 +155,18 @@ __host__ __device__ __forceinline__ size_t sign_tile_word(long r, long q, long n
 // per row).  Lane (row, g) loads words 32 P + 8 g .. + 7 of its row as two
 // 16-byte vectors from the pass's tiles (sign_tile_word: the wave's 8 KB of
 // the pair are consecutive); super-block S = 2 P + s takes words
-// 32 P + 8 g + 4 s + u, u = 0..3.  For word u and
-// half h (0, 1) the A operand is the four dwords (word >> (4 h + j)) &
-// 0x01010101, j = 0..3, so byte i of dword j is bit 8 i + 4 h + j:
-// k = 32 (32 P + 8 g + 4 s + u) + 8 i + 4 h + j.  The B operand of (S, u, h)
-// is stored in exactly that order (sign_bfrag_offset), 1 KB per MFMA, 8 KB
-// per super-block, so the expansion of the bits costs two VALU operations
-// per 4 entries and no lane exchange.
+// 32 P + 8 g + 4 s + u, u = 0..3.  For bit j = 0..3 of half h = 0, 1 the A
+// operand is the four dwords (word u >> 4 h) & (0x01010101 << j): byte i of
+// dword u is 2^j times bit 8 i + 4 h + j, k = 32 (32 P + 8 g + 4 s + u) + 8 i
+// + 4 h + j.  The bits are not moved to the bytes' low end (that costs a shift
+// per dword more): the four j accumulate apart, each a sum times 2^j, at most
+// 2^3 2^7 2^20 / 4 < 2^29, and are shifted and added once at the end.  The B
+// operand of (S, j, h) is stored in exactly that order (sign_bfrag_offset),
+// 1 KB per MFMA, 8 KB per super-block, so the expansion of the bits costs a
+// little over one VALU operation per 4 entries and no lane exchange.
 // ---------------------------------------------------------------------
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 // Register sets of the pass's ring: one pair in use, kSignPF - 1 in flight.
-// 2 sets: 124 VGPRs (the occupancy query reports 3 workgroups per CU); 3
-// sets (fewer waves per SIMD, about the same bytes in flight per SIMD) ran
-// 4% slower at N = K = 10^5.
 constexpr int kSignPF = 2;
 
 template <int I, int U, class F> __device__ __forceinline__ void sign_unroll(F &&f) {
@@ -188,7 +188,7 @@ __device__ __forceinline__ size_t sign_bfrag_offset(long k, int c) {
   const long S = 2 * (q >> 5) + ((q >> 2) & 1);
   const int g = (int)((q >> 3) & 3), u = (int)(q & 3);
   const int b = (int)(k & 31), i = b >> 3, h = (b >> 2) & 1, j = b & 3;
-  return ((((size_t)S * 4 + u) * 2 + h) * 64 + (c + 16 * g)) * 16 + j * 4 + i;
+  return ((((size_t)S * 4 + j) * 2 + h) * 64 + (c + 16 * g)) * 16 + u * 4 + i;
 }
 
 // The 7 signed base-256 digits of round(v 2^54), |v| <= 1: e = d + bias is
@@ -227,113 +227,151 @@ __global__ __launch_bounds__(kBlock) void sign_limbs_kernel(const R *__restrict_
   for (int c = 0; c < 16; ++c) bfrag[sign_bfrag_offset(k, c)] = d[c];
 }
 
-__device__ __forceinline__ i32x4_t sign_expand(uint32_t w, int h) {
-  const uint32_t x = w >> (4 * h), m = 0x01010101u;
-  return i32x4_t{(int)(x & m), (int)((x >> 1) & m), (int)((x >> 2) & m), (int)((x >> 3) & m)};
+// The line of `units` (row group, pair) units over G workgroups: workgroup b
+// owns [sign_first_unit(b), sign_first_unit(b + 1)); the owner of unit u.
+__host__ __device__ __forceinline__ long sign_first_unit(long b, long units, long G) { return b * units / G; }
+__host__ __device__ __forceinline__ long sign_unit_owner(long u, long units, long G) { return ((u + 1) * G - 1) / units; }
+
+// The A operand of class (j, h): bit 4 h + j of every byte of the lane's four
+// words, kept in place after the shift by 4 h, so every byte is 0 or 2^j.
+__device__ __forceinline__ i32x4_t sign_class(const u32x4 w, int j, int h) {
+  const uint32_t m = 0x01010101u << j;
+  return i32x4_t{(int)((w.x >> (4 * h)) & m), (int)((w.y >> (4 * h)) & m), (int)((w.z >> (4 * h)) & m),
+                 (int)((w.w >> (4 * h)) & m)};
 }
 
-// One pass: part[sp][r][c] = sum over the k of split sp of bit(r, k) * B[k][c]
-// for the rows r < ldp of the pass's tiles (its bit rows, then the ones row:
-// T_c = sum_k B[k][c], then zero rows).  A workgroup = 4 waves on the same
-// split of super-block pairs; wave w owns row group 4 (group of blocks) + w,
-// NT 16-row tiles.  The B fragments of a pair (16 KB) are loaded once per
-// workgroup, 64 bytes per thread, and shared through LDS (double-buffered,
-// one barrier per pair); every thread's loads for pair P + kSignPF (its
-// share of the B fragments before the MFMAs of pair P, its rows' bit words
-// after them) are issued in the order they are used, so kSignPF - 1 pairs
-// stay in flight behind the one in use.
+// One pass: part[sp][r][c] = the sum of slot sp's share of k over bit(r, k) *
+// B[k][c], for the rows r < ldp of the pass's tiles (its bit rows, then the
+// ones row: T_c = sum_k B[k][c], then zero rows).  The work is a line of
+// units (row group of 256 rows, pair of super-blocks), row group major, cut
+// into gridDim.x equal stretches: a workgroup takes its stretch in order and
+// writes its sums whenever a row group or the stretch ends, into the slot
+// that counts the workgroups of that row group (sums are exact integers, so
+// the cut does not change a result; slots that a row group does not reach
+// stay zero).  Equal stretches because no split count fits every size: one
+// (row group, range of k) per workgroup left 1.53 rounds of resident
+// workgroups at N = K = 10^5.
+// A workgroup = 4 waves, wave w on NT 16-row tiles of the row group.  The B
+// fragments of a pair (16 KB) are loaded once per workgroup, 64 bytes per
+// thread, and shared through LDS (double-buffered, one barrier per pair);
+// every thread's loads for pair P + kSignPF (its share of the B fragments
+// before the MFMAs of pair P, its rows' bit words after them) are issued in
+// the order they are used, so kSignPF - 1 pairs stay in flight behind the one
+// in use.
+// Bound: the stream of bits (1.25 GB per pass at N = K = 10^5) together with
+// VALU issue.  With the bits expanded to bytes 0 / 1 (7.5 instructions per
+// MFMA, VALU busy 61% of the time) a pass took 249 us, 5.0 TB/s; leaving each
+// bit at its place (4.5 instructions, four accumulator sets, 231 VGPRs, 2
+// waves per SIMD), a row group's pair 32 KB of consecutive memory and equal
+// stretches: 233 us, 5.4 TB/s.  One right-hand side: 527 -> 497 us; N = K =
+// 65535 245 -> 223; an attempt at N = K = 10^4 is unchanged by this kernel
+// (400 units, 7.5 us, latency).
 template <class R, int NT>
-__global__ __launch_bounds__(kBlock) void sign_mfma_kernel(const u32x4 *__restrict__ tiles,
-                                                            const u32x4 *__restrict__ bfrag, long npairs,
-                                                            long pairs_per, int nsplit, int32_t *__restrict__ part,
-                                                            long ldp, const State<R> *st, int check_state) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void sign_mfma_kernel(
+    const u32x4 *__restrict__ tiles, const u32x4 *__restrict__ bfrag, int npairs, long units,
+    int32_t *__restrict__ part, long ldp, const State<R> *st, int check_state) {
   constexpr int NW = kBlock / kWave;
   constexpr int BPT = 2 * 8 * kWave / kBlock;  // 16-byte B pieces per thread and pair
   __shared__ u32x4 bsh[2][2 * 8 * kWave];
   if (check_state && (!st->active || st->commit_pending)) return;
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const long rgb = blockIdx.x / nsplit;  // the workgroup's 4 row groups
-  const int sp = (int)(blockIdx.x % nsplit);
-  const long rg = rgb * NW + wave;
-  const long p0 = (long)sp * pairs_per, p1 = p0 + pairs_per < npairs ? p0 + pairs_per : npairs;
+  const long G = gridDim.x, u0 = sign_first_unit(blockIdx.x, units, G), u1 = sign_first_unit(blockIdx.x + 1, units, G);
+  if (u0 >= u1) return;
   const int g = lane >> 4, rl = lane & 15;
   static_assert(NT == 4, "tile order: 64 rows per wave");
-  // the wave's 8 KB of pair P start at tw + 512 P (16-byte slots); every
+  // the wave's 8 KB of unit u start at tw + 2048 u (16-byte slots); every
   // lane loads (no divergent branch around the loads, which would make the
   // compiler wait for every load in flight)
-  const u32x4 *tw = tiles + (size_t)rg * npairs * 512 + lane;
-  i32x4_t acc[NT];
+  const u32x4 *tw = tiles + (size_t)wave * 512 + lane;
+  i32x4_t acc[4][NT];  // [j]: sums with bits as 2^j
+  auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = i32x4_t{0, 0, 0, 0};
-  // pair P: the rows' bit words and this thread's pieces of the pair's B
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[j][t] = i32x4_t{0, 0, 0, 0};
+  };
+  // unit u: the rows' bit words; pair P: this thread's pieces of the pair's B
   // fragments (piece f = tid + kBlock j of the pair's 1024, in the pair's
-  // order: super-block s, (u, h), lane).  Nothing here consumes a value.
-  auto load_w = [&](long P, u32x4 (&W)[NT][2]) {
+  // order: super-block s, (j, h), lane).  Nothing here consumes a value.
+  auto load_w = [&](long u, u32x4 (&W)[NT][2]) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      W[t][0] = tw[(size_t)P * 512 + (2 * t) * 64];
-      W[t][1] = tw[(size_t)P * 512 + (2 * t + 1) * 64];
+      W[t][0] = tw[(size_t)u * NW * 512 + (2 * t) * 64];
+      W[t][1] = tw[(size_t)u * NW * 512 + (2 * t + 1) * 64];
     }
   };
-  auto load_b = [&](long P, u32x4 (&Bst)[BPT]) {
+  auto load_b = [&](int P, u32x4 (&Bst)[BPT]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < BPT; ++j) Bst[j] = bfrag[(size_t)P * 2 * 8 * kWave + tid + kBlock * j];
   };
-  // the MFMAs of super-block 2 P + s, B fragments from LDS buffer buf
-  auto multiply = [&](const u32x4 (&W)[NT][2], int s, int buf) {
+  // the MFMAs of super-block s of a pair, B fragments from LDS buffer buf
+  auto multiply = [&](const u32x4 (&W)[NT][2], int s, int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const i32x4_t b = __builtin_bit_cast(i32x4_t, bsh[buf][(s * 8 + u * 2 + h) * kWave + lane]);
+      for (int j = 0; j < 4; ++j) {
+        const i32x4_t b = __builtin_bit_cast(i32x4_t, bsh[buf][(s * 8 + j * 2 + h) * kWave + lane]);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-          acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(sign_expand(W[t][s][u], h), b, acc[t], 0, 0, 0);
+          acc[j][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(sign_class(W[t][s], j, h), b, acc[j][t], 0, 0, 0);
       }
   };
-  // Ring of kSignPF register sets, slot d holding pair P + d.  Loads past
-  // the split's end re-read its last pair (harmless, and no branch).
-  const long plast = p1 - 1;
-  auto cl = [](long x, long hi) { return x < hi ? x : hi; };
+  // One row group's part of the stretch at a time, pairs [p0, p1).  Ring of
+  // kSignPF register sets, slot d holding pair P + d; loads past the end
+  // re-read the last pair (harmless, and no branch).  (Carrying the ring over
+  // into the next row group, with the sums written inside the pair loop, was
+  // 6% slower per pair.)
   u32x4 W[kSignPF][NT][2], Bst[kSignPF][BPT];
-  if (p0 < p1)
-    sign_unroll<0, kSignPF>([&](auto i) {
+#pragma unroll 1
+  for (long u = u0; u < u1;) {
+    const long rgb = u / npairs, base = rgb * npairs;
+    const int p0 = (int)(u - base), p1 = u1 - base < npairs ? (int)(u1 - base) : npairs, plast = p1 - 1;
+    auto cl = [&](int p) __attribute__((always_inline)) { return p < plast ? p : plast; };
+    sign_unroll<0, kSignPF>([&](auto i) __attribute__((always_inline)) {
       constexpr int d = decltype(i)::value;
-      load_b(cl(p0 + d, plast), Bst[d]);
-      load_w(cl(p0 + d, plast), W[d]);
+      load_b(cl(p0 + d), Bst[d]);
+      load_w(base + cl(p0 + d), W[d]);
     });
-  // pair P + d from slot d: its B fragments to LDS and a barrier, the slot's
-  // B pieces refilled with pair P + d + kSignPF, the pair's MFMAs, then the
-  // slot's bit words refilled (after the MFMAs that read them)
-  auto pair = [&](auto i, long P, bool refill) {
-    constexpr int d = decltype(i)::value;
-    const int buf = (int)((P + d - p0) & 1);
+    clear();
+    // pair P + d from slot d: its B fragments to LDS and a barrier, the slot's
+    // B pieces refilled with pair P + d + kSignPF, the pair's MFMAs, then the
+    // slot's bit words refilled (after the MFMAs that read them)
+    auto pair = [&](auto i, int P, bool refill) __attribute__((always_inline)) {
+      constexpr int d = decltype(i)::value;
+      const int buf = (P + d - p0) & 1;
 #pragma unroll
-    for (int j = 0; j < BPT; ++j) bsh[buf][tid + kBlock * j] = Bst[d][j];
-    __syncthreads();
-    if (refill) load_b(cl(P + d + kSignPF, plast), Bst[d]);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(W[d], 0, buf);
-    multiply(W[d], 1, buf);
-    __builtin_amdgcn_sched_barrier(0);
-    if (refill) load_w(cl(P + d + kSignPF, plast), W[d]);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  long P = p0;
-  for (; P + kSignPF <= p1; P += kSignPF) sign_unroll<0, kSignPF>([&](auto i) { pair(i, P, true); });
-  sign_unroll<0, kSignPF - 1>([&](auto i) {
-    if (P + decltype(i)::value < p1) pair(i, P, false);
-  });
+      for (int j = 0; j < BPT; ++j) bsh[buf][tid + kBlock * j] = Bst[d][j];
+      __syncthreads();
+      if (refill) load_b(cl(P + d + kSignPF), Bst[d]);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(W[d], 0, buf);
+      multiply(W[d], 1, buf);
+      __builtin_amdgcn_sched_barrier(0);
+      if (refill) load_w(base + cl(P + d + kSignPF), W[d]);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    int P = p0;
+    for (; P + kSignPF <= p1; P += kSignPF)
+      sign_unroll<0, kSignPF>([&](auto i) __attribute__((always_inline)) { pair(i, P, true); });
+    sign_unroll<0, kSignPF - 1>([&](auto i) __attribute__((always_inline)) {
+      if (P + decltype(i)::value < p1) pair(i, P, false);
+    });
+    __syncthreads();  // the next row group starts at buffer 0 again
+    const long slot = blockIdx.x - sign_unit_owner(base, units, G);
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const long r = rg * 16 * NT + 16 * t + 4 * g + v;
-      part[((size_t)sp * ldp + r) * 16 + rl] = acc[t][v];
-    }
+      for (int v = 0; v < 4; ++v) {
+        const long r = (rgb * NW + wave) * 16 * NT + 16 * t + 4 * g + v;
+        // acc[j] is 2^j times its classes' sum: exact shifts
+        part[((size_t)slot * ldp + r) * 16 + rl] =
+            acc[0][t][v] + (acc[1][t][v] >> 1) + (acc[2][t][v] >> 2) + (acc[3][t][v] >> 3);
+      }
+    u = base + p1;
+  }
 }
 
-// The 14 digit sums of row r (2 P - T over the splits), exact in int64.
+// The 14 digit sums of row r (2 P - T over the slots), exact in int64.
 __device__ __forceinline__ void sign_row_sums(const int32_t *__restrict__ part, int nsplit, long ldp, long r,
                                               long trow, long long (&sc)[7], long long (&ss)[7]) {
 #pragma unroll
