@@ -113,7 +113,8 @@ template <class R> struct Engine : EngineBase {
     int wgs = 1;          // workgroups that share the units
     int nsplit = 1;       // most workgroups of one row group: slots of part
     uint32_t *tiles = nullptr;
-    uint8_t *bfrag = nullptr;
+    uint8_t *bfrag = nullptr;      // owns bfrag_rhs and part too
+    uint8_t *bfrag_rhs = nullptr;  // pass 1: the vector of a stand-alone right-hand side
     int32_t *part = nullptr;
     uint32_t *ones = nullptr;  // the ones row: bits set for k < kdim, 16 nsb words
   } s_pass[2];
@@ -619,8 +620,7 @@ template <class R> struct Engine : EngineBase {
   }
 
   void drop_sign() {
-    void *b[] = {s_pass[0].tiles, s_pass[0].bfrag, s_pass[0].part, s_pass[0].ones,
-                 s_pass[1].tiles, s_pass[1].bfrag, s_pass[1].part, s_pass[1].ones};
+    void *b[] = {s_pass[0].tiles, s_pass[0].bfrag, s_pass[0].ones, s_pass[1].tiles, s_pass[1].bfrag, s_pass[1].ones};
     for (void *p : b)
       if (p) (void)hipFree(p);
     s_pass[0] = s_pass[1] = SignPass();
@@ -649,10 +649,14 @@ template <class R> struct Engine : EngineBase {
     return p;
   }
   int alloc_sign_pass(SignPass &p, long kdim) {
-    HIP_TRY(hipMalloc((void **)&p.bfrag, (size_t)p.nsb * 8 * kWave * 16));
-    // slots that a row group does not reach stay as cleared here
-    HIP_TRY(hipMalloc((void **)&p.part, sizeof(int32_t) * 16 * (size_t)p.nsplit * p.ldp));
-    HIP_TRY(hipMemsetAsync(p.part, 0, sizeof(int32_t) * 16 * (size_t)p.nsplit * p.ldp, stream));
+    // one allocation, cleared once: columns past the vectors' end and slots
+    // that a row group does not reach stay zero
+    const size_t frag_bytes = (size_t)p.nsb * 8 * kWave * 16, nfrag = &p == &s_pass[0] ? 2 : 1;
+    const size_t part_bytes = sizeof(int32_t) * 16 * (size_t)p.nsplit * p.ldp;
+    HIP_TRY(hipMalloc((void **)&p.bfrag, nfrag * frag_bytes + part_bytes));
+    HIP_TRY(hipMemsetAsync(p.bfrag, 0, nfrag * frag_bytes + part_bytes, stream));
+    if (nfrag == 2) p.bfrag_rhs = p.bfrag + frag_bytes;
+    p.part = (int32_t *)(p.bfrag + nfrag * frag_bytes);
     std::vector<uint32_t> ones((size_t)16 * p.nsb, 0u);
     for (long q = 0; q < (long)ones.size(); ++q)
       ones[q] = 32 * (q + 1) <= kdim ? 0xFFFFFFFFu : (32 * q < kdim ? (1u << (kdim - 32 * q)) - 1u : 0u);
@@ -1008,24 +1012,30 @@ template <class R> struct Engine : EngineBase {
     }
   }
 
-  // packed sign factor: the stage vectors as digits, pass 1 over bitsT
-  // (rows m), G as digits, pass 2 over bits (rows n), sums + stage epilogue
+  bool sign_path() const { return factored && sign; }
+  unsigned vec_blocks(long n) const { return (unsigned)((n + kBlock - 1) / kBlock); }
+  void launch_sign_limbs(const R *cs_in, uint8_t *bfrag) {
+    if (K > 0) sign_limbs_kernel<R><<<vec_blocks(N), kBlock, 0, stream>>>(cs_in, cs_in + ldv, N, bfrag);
+  }
+  // packed sign factor: pass 1 (rows m) over the vector's digits, G as digits,
+  // pass 2 (rows n), sums + stage epilogue.  An attempt's stages find their
+  // vector's digits in the pass's own buffer (from the launch that wrote the
+  // vector); a stand-alone right-hand side makes them in its own.
   template <int KIND> void launch_sign(const Vecs<R> &v) {
-    const int chk = v.check_state && KIND >= 2;
+    const bool attempt = v.check_state && KIND >= 2;
+    const int chk = attempt;
     const SignPass &p1 = s_pass[0], &p2 = s_pass[1];
     if (K > 0) {
-      const long n_pad = p1.nsb * kSignSB, k_pad = p2.nsb * kSignSB;
-      sign_limbs_kernel<R><<<(unsigned)((n_pad + kBlock - 1) / kBlock), kBlock, 0, stream>>>(
-          v.cs_in, v.cs_in + ldv, N, n_pad, p1.bfrag, st, chk);
+      uint8_t *vec = attempt ? p1.bfrag : p1.bfrag_rhs;
+      if (!attempt) launch_sign_limbs(v.cs_in, vec);
       sign_mfma_kernel<R, kSignNT><<<(unsigned)p1.wgs, kBlock, 0, stream>>>(
-          (const u32x4 *)p1.tiles, (const u32x4 *)p1.bfrag, (int)p1.npairs, p1.units, p1.part, p1.ldp, st, chk);
-      sign_gram_kernel<R><<<(unsigned)((k_pad + kBlock - 1) / kBlock), kBlock, 0, stream>>>(
-          p1.part, p1.nsplit, p1.ldp, w, K, k_pad, p2.bfrag, st, chk);
+          (const u32x4 *)p1.tiles, (const u32x4 *)vec, (int)p1.npairs, p1.units, p1.part, p1.ldp, st, chk);
+      sign_gram_kernel<R><<<vec_blocks(K), kBlock, 0, stream>>>(p1.part, p1.nsplit, p1.ldp, w, K, p2.bfrag, st, chk);
       sign_mfma_kernel<R, kSignNT><<<(unsigned)p2.wgs, kBlock, 0, stream>>>(
           (const u32x4 *)p2.tiles, (const u32x4 *)p2.bfrag, (int)p2.npairs, p2.units, p2.part, p2.ldp, st, chk);
     }
-    sign_stage_kernel<R, KIND><<<(unsigned)((N + kBlock - 1) / kBlock), kBlock, 0, stream>>>(
-        p2.part, K > 0 ? p2.nsplit : 0, p2.ldp, v);
+    sign_stage_kernel<R, KIND><<<vec_blocks(N), kBlock, 0, stream>>>(p2.part, K > 0 ? p2.nsplit : 0, p2.ldp, v,
+                                                                     attempt && K > 0 ? p1.bfrag : nullptr);
   }
 
   template <int KIND> void launch_factored(const Vecs<R> &v) {
@@ -1197,13 +1207,16 @@ template <class R> struct Engine : EngineBase {
         lowrank_emit_kernel<R, decltype(kt)::value, decltype(exact)::value>
             <<<(unsigned)lr_grid, lr_threads, 0, stream>>>(emit_args(), lr_args(0, 0));
       });
+    else if (sign_path() && K > 0)
+      sign_emit_kernel<R><<<(unsigned)nblk_emit, kBlock, 0, stream>>>(emit_args(), s_pass[0].bfrag);
     else
       emit_commit_kernel<R><<<(unsigned)nblk_emit, kBlock, 0, stream>>>(emit_args());
   }
-  // Before the first attempt after a change of coupling: the low-rank path's
-  // partials of the pending stage-2 vector
+  // Before the first attempt after a change of coupling: what its paths keep
+  // of the pending stage-2 vector (the low-rank partials, the signs' digits)
   void launch_prepare() {
     if (lr_path()) launch_gram(cs[0], 0);
+    if (sign_path()) launch_sign_limbs(cs[0], s_pass[0].bfrag);
   }
   // the order parameters of the last attempt's rows (earlier ones are
   // computed by the next attempt's control_kernel): before the host looks

@@ -1165,9 +1165,9 @@ template <class R> __device__ __forceinline__ R dense_value(const R Q[4], R yl, 
   return rfma<R>(hh * x, in, yl);
 }
 
-template <class R> __device__ __forceinline__ void stage2_vector(const EmitArgs<R> &a, long i, R y, R k1, R h) {
+template <class R>
+__device__ __forceinline__ void stage2_vector(const EmitArgs<R> &a, long i, R y, R k1, R h, R &c, R &s) {
   const R yt = rfma<R>(k1 * (R)tab::A[0][0], h, y);
-  R c, s;
   rsincos<R>(yt, c, s);
   a.cs_out[i] = c;
   a.cs_out[a.ldv + i] = s;
@@ -1207,18 +1207,18 @@ __device__ __forceinline__ void emit_rows(int n, bool valid, const R Q[4], R yl,
   }
 }
 
-template <class R>
-__global__ __launch_bounds__(kBlock) void emit_commit_kernel(const EmitArgs<R> a) {
+// The emit launch for oscillator i; true if the stage-2 vector was written
+// (the same for every thread), with this thread's part in c, s.
+template <class R> __device__ __forceinline__ bool emit_commit(const EmitArgs<R> &a, long i, R &c, R &s) {
   const State<R> *st = a.st;
   const int mode = st->job_mode;
-  if (mode == JOB_NONE) return;
+  if (mode == JOB_NONE) return false;
   __shared__ double sh[kEmitRows][2][kBlock];
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
   const bool valid = i < a.N;
   const R h = st->h;
   if (mode == JOB_STAGE2) {
-    if (valid) stage2_vector<R>(a, i, a.y[i], a.k[0][i], h);
-    return;
+    if (valid) stage2_vector<R>(a, i, a.y[i], a.k[0][i], h, c, s);
+    return true;
   }
   // every operand of the commit is in flight before the outputs are formed
   R yo = 0, yn = 0, k7 = 0;
@@ -1247,8 +1247,14 @@ __global__ __launch_bounds__(kBlock) void emit_commit_kernel(const EmitArgs<R> a
     a.ylast[i] = yo;
     a.y[i] = yn;
     a.k[0][i] = k7;
-    stage2_vector<R>(a, i, yn, k7, h);
+    stage2_vector<R>(a, i, yn, k7, h, c, s);
   }
+  return mode == JOB_COMMIT;
+}
+template <class R>
+__global__ __launch_bounds__(kBlock) void emit_commit_kernel(const EmitArgs<R> a) {
+  R c = 0, s = 0;
+  (void)emit_commit<R>(a, (long)blockIdx.x * kBlock + threadIdx.x, c, s);
 }
 
 // emit_commit_kernel for the low-rank path, on its grid (threads stride over

@@ -12,10 +12,11 @@
 // more row of ones (k < the pass's k range) and zero rows up to its padded
 // row count.
 //
-// Coupling (one RHS, five launches), on the int8 matrix cores with exact
-// integer sums:
-//   sign_limbs_kernel  (cos, sin)_n as 56-bit fixed point (2^-54 units) in
-//                      7 signed base-256 digits each: the B operand of pass 1
+// Coupling on the int8 matrix cores with exact integer sums, four launches
+// per stage (a stand-alone RHS: five).  (cos, sin)_n as 56-bit fixed point
+// (2^-54 units) in 7 signed base-256 digits each are the B operand of pass 1,
+// written by the launch that forms the vector (sign_stage_kernel,
+// sign_emit_kernel) or, for a given vector, by sign_limbs_kernel:
 //   sign_mfma_kernel   pass 1 over the pass-1 tiles: P_m = sum_n bit(m, n) * digit(n),
 //                      per digit and per range of n, plus T = sum_n digit(n)
 //   sign_gram_kernel   sum_n X_nm v_n = 2 P_m - T (X = 2 bit - 1) combined to
@@ -193,11 +194,42 @@ __device__ __forceinline__ size_t sign_bfrag_offset(long k, int c) {
 
 // The 7 signed base-256 digits of round(v 2^54), |v| <= 1: e = d + bias is
 // non-negative and below 2^56, and digit l = byte l of e minus 128 (as a
-// byte: byte ^ 0x80), so that d = sum_l digit_l 256^l.
-__device__ __forceinline__ void sign_digits(double v, uint8_t *out) {
-  const long long e = __double2ll_rn(v * kSignScale) + kSignBias;
+// byte: byte ^ 0x80), so that d = sum_l digit_l 256^l.  Bytes 0 .. 6 of the
+// result (byte 7 zero).
+__device__ __forceinline__ uint64_t sign_digits(double v) {
+  const uint64_t e = (uint64_t)(__double2ll_rn(v * kSignScale) + kSignBias);
+  return (e ^ 0x80808080808080ull) & 0xFFFFFFFFFFFFFFull;
+}
+
+// One k's 16 columns (digits of c in 0..6, of s in 7..13) of every thread of
+// a workgroup, k = kBlock blockIdx.x + thread, into the B fragments: through
+// LDS, so that each thread stores the 16 consecutive bytes of one (j, h,
+// column) of a 128-wide stretch of k (a byte at a time, 16 stores 16 bytes
+// apart, took most of the 4 us that a launch of its own spent on the digits
+// at N = 10^4; with them in the launch that forms the vector, and the sums'
+// 16-byte loads, an attempt there went from 237 to 212-225 us).
+__device__ __forceinline__ void sign_write_frags(double c, double s, bool zero, uint32_t (&sh)[kBlock][4],
+                                                 uint8_t *__restrict__ bfrag) {
+  const int tid = threadIdx.x;
+  uint64_t lo = 0, hi = 0;
+  if (!zero) {
+    const uint64_t dc = sign_digits(c), ds = sign_digits(s);
+    lo = dc | ds << 56;
+    hi = ds >> 8;
+  }
+  *reinterpret_cast<u32x4 *>(sh[tid]) = u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+  __syncthreads();
+  const int grp = tid >> 7, j = (tid >> 5) & 3, h = (tid >> 4) & 1, col = tid & 15;
+  const uint8_t *src = reinterpret_cast<const uint8_t *>(sh) + (grp * 128 + 4 * h + j) * 16 + col;
+  uint32_t w[4];
 #pragma unroll
-  for (int l = 0; l < 7; ++l) out[l] = (uint8_t)(((e >> (8 * l)) & 0xFF) ^ 0x80);
+  for (int u = 0; u < 4; ++u) {
+    w[u] = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[u] |= (uint32_t)src[(32 * u + 8 * i) * 16] << (8 * i);
+  }
+  const long k = (long)blockIdx.x * kBlock + grp * 128 + 4 * h + j;
+  *reinterpret_cast<u32x4 *>(bfrag + sign_bfrag_offset(k, col)) = u32x4{w[0], w[1], w[2], w[3]};
 }
 
 // sum_l s_l 256^l 2^-54 rounded once to double: |s_l| < 2^28.6, so the low
@@ -209,22 +241,16 @@ __device__ __forceinline__ double sign_combine(const long long (&s)[7]) {
   return __builtin_fma((double)hi, 0x1p32, (double)lo) * 0x1p-54;
 }
 
-// B fragments of pass 1 from the stage vector pair: one thread per k = n
-// (zero columns 14, 15 and zero rows for k >= n_used up to the padded end).
+// B fragments of pass 1 from a given vector pair: one thread per k = n (zero
+// columns 14, 15 and zero rows for k >= N up to the grid's end; past it the
+// buffer stays as cleared).
 template <class R>
-__global__ __launch_bounds__(kBlock) void sign_limbs_kernel(const R *__restrict__ vc, const R *__restrict__ vs,
-                                                             long n_used, long n_pad, uint8_t *__restrict__ bfrag,
-                                                             const State<R> *st, int check_state) {
-  if (check_state && (!st->active || st->commit_pending)) return;
+__global__ __launch_bounds__(kBlock) void sign_limbs_kernel(const R *__restrict__ vc, const R *__restrict__ vs, long N,
+                                                             uint8_t *__restrict__ bfrag) {
+  __shared__ __align__(16) uint32_t sh[kBlock][4];
   const long k = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (k >= n_pad) return;
-  uint8_t d[16] = {};
-  if (k < n_used) {
-    sign_digits((double)vc[k], d);
-    sign_digits((double)vs[k], d + 7);
-  }
-#pragma unroll
-  for (int c = 0; c < 16; ++c) bfrag[sign_bfrag_offset(k, c)] = d[c];
+  const long kk = k < N ? k : N - 1;
+  sign_write_frags((double)vc[kk], (double)vs[kk], k >= N, sh, bfrag);
 }
 
 // The line of `units` (row group, pair) units over G workgroups: workgroup b
@@ -376,49 +402,62 @@ __device__ __forceinline__ void sign_row_sums(const int32_t *__restrict__ part, 
                                               long trow, long long (&sc)[7], long long (&ss)[7]) {
 #pragma unroll
   for (int l = 0; l < 7; ++l) { sc[l] = 0; ss[l] = 0; }
+#pragma unroll 2
   for (int sp = 0; sp < nsplit; ++sp) {
-    const int32_t *pr = part + ((size_t)sp * ldp + r) * 16, *pt = part + ((size_t)sp * ldp + trow) * 16;
+    const i32x4_t *pr = reinterpret_cast<const i32x4_t *>(part + ((size_t)sp * ldp + r) * 16);
+    const i32x4_t *pt = reinterpret_cast<const i32x4_t *>(part + ((size_t)sp * ldp + trow) * 16);
+    int32_t p[16], t[16];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const i32x4_t x = pr[q], y = pt[q];
+      p[4 * q] = x.x, p[4 * q + 1] = x.y, p[4 * q + 2] = x.z, p[4 * q + 3] = x.w;
+      t[4 * q] = y.x, t[4 * q + 1] = y.y, t[4 * q + 2] = y.z, t[4 * q + 3] = y.w;
+    }
 #pragma unroll
     for (int l = 0; l < 7; ++l) {
-      sc[l] += 2LL * pr[l] - pt[l];
-      ss[l] += 2LL * pr[7 + l] - pt[7 + l];
+      sc[l] += 2LL * p[l] - t[l];
+      ss[l] += 2LL * p[7 + l] - t[7 + l];
     }
   }
 }
 
 // G_m = w_m sum_n X_nm (cos, sin)_n from the pass-1 sums, written as the B
-// fragments of pass 2 (one thread per k = m, zero past K up to the padded end).
+// fragments of pass 2 (one thread per k = m, zero past K).
 template <class R>
 __global__ __launch_bounds__(kBlock) void sign_gram_kernel(const int32_t *__restrict__ part, int nsplit, long ldp,
-                                                            const R *__restrict__ w, long K, long k_pad,
+                                                            const R *__restrict__ w, long K,
                                                             uint8_t *__restrict__ bfrag, const State<R> *st,
                                                             int check_state) {
   if (check_state && (!st->active || st->commit_pending)) return;
+  __shared__ __align__(16) uint32_t sh[kBlock][4];
   const long m = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (m >= k_pad) return;
-  uint8_t d[16] = {};
+  double c = 0.0, s = 0.0;
   if (m < K) {
     long long sc[7], ss[7];
-    sign_row_sums(part, nsplit, ldp, m, K, sc, ss);
     const double wm = (double)w[m];
-    sign_digits(sign_combine(sc) * wm, d);
-    sign_digits(sign_combine(ss) * wm, d + 7);
+    sign_row_sums(part, nsplit, ldp, m, K, sc, ss);
+    c = sign_combine(sc) * wm;
+    s = sign_combine(ss) * wm;
   }
-#pragma unroll
-  for (int c = 0; c < 16; ++c) bfrag[sign_bfrag_offset(m, c)] = d[c];
+  sign_write_frags(c, s, m >= K, sh, bfrag);
 }
 
-// C_n, S_n from the pass-2 sums, then the stage epilogue of row n; stage 7
-// writes one error partial per workgroup.
+// C_n, S_n from the pass-2 sums, then the stage epilogue of row n; stages 2..6
+// also write the digits of their output vector (the next pass 1's B operand),
+// stage 7 one error partial per workgroup.
 template <class R, int KIND>
 __global__ __launch_bounds__(kBlock) void sign_stage_kernel(const int32_t *__restrict__ part, int nsplit, long ldp,
-                                                             Vecs<R> v) {
+                                                             Vecs<R> v, uint8_t *__restrict__ bfrag) {
+  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
+  // the epilogue's operands are in flight before the state check and the sums
+  const RowOps<R, KIND> ops = row_load<R, KIND>(v, i < v.N ? i : v.N - 1);
+  asm volatile("" ::: "memory");
   if constexpr (KIND >= 2) {
     if (v.check_state && (!v.st->active || v.st->commit_pending)) return;
   }
   __shared__ double errsq[kBlock];
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
   double sq = 0.0;
+  R c = 0, s = 0;
   if (i < v.N) {
     double C = 0.0, S = 0.0;
     if (nsplit > 0) {
@@ -427,12 +466,25 @@ __global__ __launch_bounds__(kBlock) void sign_stage_kernel(const int32_t *__res
       C = sign_combine(sc);
       S = sign_combine(ss);
     }
-    sq = row_epilogue<R, KIND>(v, i, (R)C, (R)S);
+    sq = row_finish<R, KIND>(v, i, ops, (R)C, (R)S, &c, &s);
+  }
+  if constexpr (KIND >= 2 && KIND < 7) {
+    __shared__ __align__(16) uint32_t sh[kBlock][4];
+    if (bfrag) sign_write_frags((double)c, (double)s, i >= v.N, sh, bfrag);
   }
   if constexpr (KIND == 7) {
     const double tot = block_sum(sq, errsq);
     if (threadIdx.x == 0) v.err_part[blockIdx.x] = tot;
   }
+}
+
+// emit_commit_kernel that also writes the digits of the stage-2 vector.
+template <class R>
+__global__ __launch_bounds__(kBlock) void sign_emit_kernel(const EmitArgs<R> a, uint8_t *__restrict__ bfrag) {
+  __shared__ __align__(16) uint32_t sh[kBlock][4];
+  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
+  R c = 0, s = 0;
+  if (emit_commit<R>(a, i, c, s)) sign_write_frags((double)c, (double)s, i >= a.N, sh, bfrag);
 }
 
 // Dense rows from the packed signs with the dense generator's chain
