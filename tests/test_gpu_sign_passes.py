@@ -36,3 +36,29 @@ def test_sign_passes_cut(km, orc, N, K, prec):
     tol = (2.0**-22 if prec == "f32" else 1e-13) * (np.abs(omega.astype(np.float64)) + c1 * K)
     assert np.all(np.abs(f.astype(np.float64) - fo) <= tol)
     assert np.all(np.abs(cp.astype(np.float64) - cso) <= np.repeat(tol, 2))
+
+
+@pytest.mark.parametrize("N,K", [(255, 257), (513, 1100)])
+def test_sign_attempts_with_right_hand_sides_between(km, N, K):
+    """The digits of an attempt's vectors are written by the launches that form
+    them and stay valid while stand-alone right-hand sides of other phases run
+    in between: the same bits as without them."""
+    rng = np.random.default_rng(N)
+    omega = rng.standard_normal(N).astype(np.float32)
+    theta = rng.uniform(-3, 3, N).astype(np.float32)
+    out = []
+    for between in (False, True):
+        print(f"case sign attempts N={N} K={K} between={between}", flush=True)
+        with km.Integrator(N, km.F32, atol=1e-7, c1=2.0) as it:
+            it.set_omega(omega)
+            it.set_factor_sign(K, 5)
+            it.use_factored(True)
+            it.set_state(theta, 0.0, 1e-3)
+            it.begin(np.zeros(0), 10.0)
+            for _ in range(4):
+                if between:
+                    it.rhs(theta[::-1].copy())
+                status = it.advance(5)
+            out.append((it.get_state()[0], status.accepted, it.rhs(theta)))
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+    assert np.array_equal(out[0][2], out[1][2])
