@@ -705,13 +705,32 @@ __global__ __launch_bounds__(kBlock) void rebuild_stage_kernel(const RebuildArgs
   Acc accC[ROWS], accS[ROWS];
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) { accC[r] = 0; accS[r] = 0; }
-  for (long c = (long)threadIdx.x * VEC; c < ldv; c += STRIDE) {
+  struct Chunk {
     R cv[VEC], sv[VEC], xj[KT][VEC];
-    load_reals<R, VEC>(cosv + c, cv);
-    load_reals<R, VEC>(sinv + c, sv);
+  };
+  auto load = [&](long c, Chunk &ch) __attribute__((always_inline)) {
+    load_reals<R, VEC>(cosv + c, ch.cv);
+    load_reals<R, VEC>(sinv + c, ch.sv);
 #pragma unroll
     for (int m = 0; m < KT; ++m)
-      if (m < K) load_reals<R, VEC>(a.XT + m * ldv + c, xj[m]);
+      if (m < K) load_reals<R, VEC>(a.XT + m * ldv + c, ch.xj[m]);
+  };
+  // The next chunk's loads ahead of this one's products in the FP32 K = 5 form
+  // (222 registers, 2 waves per SIMD either way): N = 200000 11.52 -> 10.88 ms,
+  // N = 20000 151 -> 134 us, N = 60000 1049 -> 1006.  The others lose a wave or
+  // spill into AGPRs for it: FP64 K = 5, N = 60000 1742 -> 1809 us; FP32 K = 8,
+  // N = 20000 266 -> 282; FP64 K = 8 541 -> 628.
+  constexpr bool AHEAD = EXACT && sizeof(R) == 4;
+  long c = (long)threadIdx.x * VEC;
+  Chunk cur, nxt;
+  if (AHEAD && c < ldv) load(c, cur);
+  for (; c < ldv; c += STRIDE) {
+    if constexpr (AHEAD) {
+      load(c + STRIDE < ldv ? c + STRIDE : c, nxt);
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      load(c, cur);
+    }
 #pragma unroll
     for (int r = 0; r < ROWS; ++r)
 #pragma unroll
@@ -719,10 +738,11 @@ __global__ __launch_bounds__(kBlock) void rebuild_stage_kernel(const RebuildArgs
         R mij = 0;
 #pragma unroll
         for (int m = 0; m < KT; ++m)
-          if (m < K) mij = rfma<R>(wm[m], xi[r][m] * xj[m][q], mij);
-        accC[r] = rfma<Acc>((Acc)mij, (Acc)cv[q], accC[r]);
-        accS[r] = rfma<Acc>((Acc)mij, (Acc)sv[q], accS[r]);
+          if (m < K) mij = rfma<R>(wm[m], xi[r][m] * cur.xj[m][q], mij);
+        accC[r] = rfma<Acc>((Acc)mij, (Acc)cur.cv[q], accC[r]);
+        accS[r] = rfma<Acc>((Acc)mij, (Acc)cur.sv[q], accS[r]);
       }
+    if constexpr (AHEAD) cur = nxt;
   }
   finish_rows<R, Acc, ROWS, KIND>(accC, accS, row0, (R)1, a.v);
 }
