@@ -782,8 +782,8 @@ __global__ __launch_bounds__(kBlock) void bemit_kernel(const BEmit a) {
     const int slot0 = in->ring_count, lo = in->pend_lo;
     emit_rows<float>(
         n_emit, valid, Q, yl, tl, hh, sh, [&](int q) { return a.t_eval[lo + q]; }, [](int, float) {},
-        [&](int q) {
-          return reinterpret_cast<double2 *>(a.ord_part) + ((size_t)b * a.ring_cap + slot0 + q) * a.nblk + blockIdx.x;
+        [&](int q, double2 sums) {
+          reinterpret_cast<double2 *>(a.ord_part)[((size_t)b * a.ring_cap + slot0 + q) * a.nblk + blockIdx.x] = sums;
         });
   }
   if (n_emit == pend && valid) {

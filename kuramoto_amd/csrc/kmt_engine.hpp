@@ -101,7 +101,7 @@ template <class R> struct Engine : EngineBase {
   int2 *sym_ij = nullptr;
   SymPair<double> *sym_prow = nullptr, *sym_pcol = nullptr;
   double *lr_part = nullptr, *lr_G = nullptr;
-  int lr_nblk = 0, lr_grid = 0, lr_threads = kBlock;
+  int lr_nblk = 0, lr_blocks = 0;
   // packed +-1 factor (kmt_set_factor_sign): per pass (1: rows m over
   // k = n, 2: rows n over k = m) the sign bits in the pass's tile order
   // (ldp rows of 32 npairs words: the bit rows, the ones row, zero rows),
@@ -595,13 +595,8 @@ template <class R> struct Engine : EngineBase {
       HIP_TRY(hipMemcpyAsync(w, wv, sizeof(R) * K, hipMemcpyHostToDevice, stream));
     }
     lr_nblk = (int)std::min<long>((N + kBlock - 1) / kBlock, 512);
-    // one row per thread, the workgroups spread over the CUs once
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) cus = 1;
-    lr_threads = (int)std::min<long>(std::max<long>(round_up((N + cus - 1) / cus, kWave), kBlock),
-                                     lr_max_threads(sizeof(R), lr_rank_bound()));
-    lr_grid = (int)std::min<long>((N + lr_threads - 1) / lr_threads, kLrMaxBlocks);
-    const int nparts = std::max(lr_nblk, 3 * lr_grid);
+    lr_blocks = (int)std::min<long>((N + kBlock - 1) / kBlock, kLrMaxBlocks);
+    const int nparts = std::max(lr_nblk, 3 * lr_blocks);
     if (K <= kLrMaxRank) {
       KMT_TRY(alloc_vec(&XT, (long)kk * ldv));
       transpose_factor_kernel<R><<<(unsigned)((N + kBlock - 1) / kBlock), kBlock, 0, stream>>>(X, K, N, ldv, XT);
@@ -945,19 +940,20 @@ template <class R> struct Engine : EngineBase {
   // partial-sum buffers of the fused low-rank path: 0 and 1 alternate between
   // the stages of an attempt (0: also the stage-2 vector's, kept between
   // attempts), 2 belongs to stand-alone right-hand sides
-  double *lr_p(int which) const { return lr_part + (size_t)which * 2 * std::max(K, 1) * lr_grid; }
+  double *lr_p(int which) const { return lr_part + (size_t)which * 2 * std::max(K, 1) * lr_blocks; }
   LrArgs<R> lr_args(int pin, int pout) const {
     LrArgs<R> l;
     l.XT = XT;
     l.w = w;
     l.K = K;
+    l.blocks = lr_blocks;
     l.part_in = lr_p(pin);
-    l.nparts = lr_grid;
     l.part_out = lr_p(pout);
     return l;
   }
-  // the rank bound of the kernels that lr_dispatch picks
-  int lr_rank_bound() const { return K <= 8 ? std::max(K, 1) : kLrMaxRank; }
+  // the launch: one block per workgroup, or two
+  int lr_threads() const { return lr_blocks > kLrPairedBlocks ? kLrThreads : kBlock; }
+  unsigned lr_grid() const { return (unsigned)(lr_blocks > kLrPairedBlocks ? (lr_blocks + 1) / 2 : lr_blocks); }
   // f(rank bound, exact) for this context's rank
   template <class F> void lr_dispatch(F &&f) {
     using std::integral_constant;
@@ -977,7 +973,7 @@ template <class R> struct Engine : EngineBase {
   void launch_gram(const R *cs_in, int pout) {
     lr_dispatch([&](auto kt, auto exact) {
       lowrank_gram_kernel<R, decltype(kt)::value, decltype(exact)::value>
-          <<<(unsigned)lr_grid, lr_threads, 0, stream>>>(lr_args(0, pout), N, cs_in, ldv);
+          <<<lr_grid(), lr_threads(), 0, stream>>>(lr_args(0, pout), N, cs_in, ldv);
     });
   }
   // stage KIND from the partials in lr_p(pin); stages 2..6 write those of
@@ -985,7 +981,7 @@ template <class R> struct Engine : EngineBase {
   template <int KIND> void launch_lr_stage(const Vecs<R> &v, int pin, int pout) {
     lr_dispatch([&](auto kt, auto exact) {
       lowrank_stage_kernel<R, KIND, decltype(kt)::value, decltype(exact)::value>
-          <<<(unsigned)lr_grid, lr_threads, 0, stream>>>(lr_args(pin, pout), v);
+          <<<lr_grid(), lr_threads(), 0, stream>>>(lr_args(pin, pout), v);
     });
   }
   // one attempt's six stages on the fused low-rank path, one launch each
@@ -1092,7 +1088,7 @@ template <class R> struct Engine : EngineBase {
 
   int n_parts_stage7() const {
     if (factored == KMT_LOWRANK_REBUILD) return (int)((N + rebuild_rows() - 1) / rebuild_rows());
-    if (factored) return lr_fused() ? lr_grid : (int)((N + kBlock - 1) / kBlock);
+    if (factored) return lr_fused() ? lr_blocks : (int)((N + kBlock - 1) / kBlock);
     if (sym()) return (int)sym_nb;
     if (tune_bal) return bal_grid;
     return (int)((N + tune_rows - 1) / tune_rows);
@@ -1196,16 +1192,14 @@ template <class R> struct Engine : EngineBase {
       }
     }
     control_kernel<R><<<1, kBlock, 0, stream>>>(st, err_part, n_parts_stage7(), N, t_eval, times, ord_part,
-                                                emit_blocks(), r_ring);
+                                                nblk_emit, r_ring);
     launch_emit();
   }
-  // workgroups of the emit launch (partials per emitted row)
-  int emit_blocks() const { return lr_path() ? lr_grid : nblk_emit; }
   void launch_emit() {
     if (lr_path())
       lr_dispatch([&](auto kt, auto exact) {
         lowrank_emit_kernel<R, decltype(kt)::value, decltype(exact)::value>
-            <<<(unsigned)lr_grid, lr_threads, 0, stream>>>(emit_args(), lr_args(0, 0));
+            <<<lr_grid(), lr_threads(), 0, stream>>>(emit_args(), lr_args(0, 0), nblk_emit);
       });
     else if (sign_path() && K > 0)
       sign_emit_kernel<R><<<(unsigned)nblk_emit, kBlock, 0, stream>>>(emit_args(), s_pass[0].bfrag);
@@ -1220,7 +1214,7 @@ template <class R> struct Engine : EngineBase {
   }
   // the order parameters of the last attempt's rows (earlier ones are
   // computed by the next attempt's control_kernel): before the host looks
-  void launch_finalize() { finalize_kernel<R><<<1, kBlock, 0, stream>>>(st, ord_part, emit_blocks(), N, r_ring); }
+  void launch_finalize() { finalize_kernel<R><<<1, kBlock, 0, stream>>>(st, ord_part, nblk_emit, N, r_ring); }
 
   // Small dense networks in the working precision: whole attempts in one
   // workgroup, as far as its registers hold the matrix.  A caller's own

@@ -824,95 +824,135 @@ __global__ __launch_bounds__(kBlock) void lowrank_expand_kernel(const R *X, int 
 // ---------------------------------------------------------------------
 // Low-rank coupling, one launch per RHS (K <= kLrMaxRank).
 //   G = w .* X^T (cos, sin) is formed in two halves: the launch that writes
-//   a stage vector also writes one partial sum of X^T (cos, sin) per
-//   workgroup (wave_reduce, then the wave sums in order); the next launch
-//   starts with every workgroup adding those partials (the same order in
-//   each, so all of them hold the same G), then computes C_i = sum_m X_im
+//   a stage vector also writes partial sums of X^T (cos, sin); the next
+//   launch starts with every workgroup adding those partials (the same order
+//   in each, so all of them hold the same G), then computes C_i = sum_m X_im
 //   G_c[m], S_i likewise and the row epilogue of its stage.  The stage-2
 //   vector's partials come from lowrank_emit_kernel; lowrank_gram_kernel
 //   writes those of a given vector (a stand-alone RHS).  No cross-workgroup
 //   synchronisation inside a launch; partial buffers alternate between
 //   consecutive launches.
+// Every sum has an order that follows from N alone (the error norm feeds the
+// step size, which feeds the phases: with fast oscillators the last bit of
+// one sum is another sequence of steps a few attempts later, so neither the
+// card's CU count nor the launch's shape may enter).  The rows are split into
+// `blocks` of kBlock lanes, at most kLrMaxBlocks, lane t of block b taking
+// rows kBlock b + t, + kBlock blocks, ...: one partial per block (its four
+// waves' sums in wave order), one error partial per block and one order
+// partial per kBlock consecutive rows (block_tree both).
 // The few MB it moves stay in the caches, so a launch is bound by latency:
-// one dependent round trip after another.  One row per thread up to
-// kLrMaxThreads x kLrMaxBlocks rows, in as few and as large workgroups as
-// still cover the CUs once (fewer partials for all of them to re-add: at
-// N=200000 241 workgroups of 832 threads, 19 KB of partials each, against
-// 512 of 256 threads that strode over 1.5 rows with 40 KB); the row's X
-// (from the transposed factor: coalesced), its epilogue operands and the
-// partials are all loaded before the first of them is needed; the rank is a
-// template argument up to 8 (no guards).  N=200000, K=5, FP32: 16.2 -> 7 us
-// per stage.
+// one dependent round trip after another.  A workgroup holds one block, or
+// two (LrPlace) once there are more blocks than a card has CUs, so that the
+// partials are read once for both and each half sums half of the values; the
+// row's X (from the transposed factor: coalesced), its epilogue operands and
+// the partials are all loaded before the first of them is needed; the rank is
+// a template argument up to 8 (no guards).  One attempt, FP32, K = 5, against
+// workgroups of one block with guarded ranks and row-major X: N = 9000 66 ->
+// 27 us, N = 100000 82 -> 35, N = 200000 109 -> 41, N = 10^6 225 -> 96; K = 16,
+// N = 200000 357 -> 74; FP64, K = 5, N = 200000 121 -> 51.
 // ---------------------------------------------------------------------
 constexpr int kLrMaxRank = 16;
 constexpr int kLrMaxBlocks = 512;
-constexpr int kLrMaxThreads = 1024;
-// larger ranks need the registers of 8 waves per CU (FP32 from 8, FP64 from 6
-// on 16 waves spill)
-constexpr int lr_max_threads(int real_bytes, int K) {
-  return K > (real_bytes == 8 ? 5 : 7) ? kLrMaxThreads / 2 : kLrMaxThreads;
-}
-template <class R, int KT> constexpr int kLrThreads = lr_max_threads(sizeof(R), KT);
+constexpr int kLrPairedBlocks = 256;       // more blocks than this: two per workgroup
+constexpr int kLrThreads = 2 * kBlock;     // at most
+constexpr int kLrBlockWaves = kBlock / kWave;
 constexpr int lr_pow2(int n) { return n <= 1 ? 1 : 2 * lr_pow2((n + 1) / 2); }
+static_assert(kLrMaxBlocks <= 2 * kBlock, "a lane adds at most two partials of a value");
 
-// A workgroup's sums of acc (2K values, interleaved c / s) -> part[q][block]
-template <class R, int KT>
-__device__ __forceinline__ void lr_write_partials(const double (&acc)[2 * KT], int K, double *part) {
+template <class R> struct LrArgs {
+  const R *XT;  // [K][ldv], zero past N
+  const R *w;   // [K]
+  int K;
+  int blocks;
+  const double *part_in;  // [2K][blocks]
+  double *part_out;       // [2K][blocks]
+};
+
+// The block of this thread's half of the workgroup: b, and with two halves
+// the other end's blocks - 1 - b (with more than one row per lane the first
+// blocks hold one row more than the last ones).
+struct LrPlace {
+  int half, tid, wave;  // thread and wave within the block
+  int blk;
+  bool live;            // an odd count leaves the last workgroup's second half empty
+  __device__ __forceinline__ LrPlace(int blocks)
+      : half((int)threadIdx.x / kBlock), tid((int)threadIdx.x % kBlock), wave(tid / kWave),
+        blk(half ? blocks - 1 - (int)blockIdx.x : (int)blockIdx.x), live(!half || blk > (int)blockIdx.x) {}
+  __device__ __forceinline__ long first(long N) const { return live ? (long)blk * kBlock + tid : N; }
+};
+
+// A block's sums of acc (2K values, interleaved c / s) -> part[q][block]
+template <int KT>
+__device__ __forceinline__ void lr_write_partials(const LrPlace &pl, const double (&acc)[2 * KT], int K, int blocks,
+                                                  double *part) {
   constexpr int NV = lr_pow2(2 * KT);
-  __shared__ double red[kLrThreads<R, KT> / kWave][NV];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, nw = blockDim.x / kWave;
+  __shared__ double red[kLrThreads / kWave][NV];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   double v[NV];
 #pragma unroll
   for (int q = 0; q < NV; ++q) v[q] = q < 2 * KT ? acc[q < 2 * KT ? q : 0] : 0.0;
   const double t = wave_reduce<double, NV>(v, lane);
   red[wave][wave_slot<NV>(lane)] = t;
   __syncthreads();
-  if ((int)threadIdx.x < 2 * K) {
-    double s = red[0][threadIdx.x];
-    for (int q = 1; q < nw; ++q) s += red[q][threadIdx.x];
-    part[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
+  if (pl.tid < 2 * K && pl.live) {
+    const int w0 = wave - pl.wave;
+    double s = red[w0][pl.tid];
+#pragma unroll
+    for (int q = 1; q < kLrBlockWaves; ++q) s += red[w0 + q][pl.tid];
+    part[(size_t)pl.tid * blocks + pl.blk] = s;
   }
 }
 
-// G (2K values, interleaved c / s) from nparts partials of each, into g
-// (LDS): one wave per value, lane l adding partials l, l + 64, ...  lr_fetch
-// issues the first kLrPre loads of the wave's first value (before the
-// launch's state check; every buffer is readable then).
-constexpr int kLrPre = 4;
-__device__ __forceinline__ void lr_fetch(const double *part, int nparts, int K, double (&pre)[kLrPre]) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+// G (2K values, interleaved c / s) from the blocks' partials, into g (LDS):
+// lane t < kBlock adds partials t and t + kBlock of a value, then the waves'
+// sums in wave order.  With two blocks per workgroup the second half's lanes
+// take values K .. 2K - 1.  lr_fetch issues the loads (before the launch's
+// state check; every buffer is readable then).
+template <class R, int KT> struct LrFetched {
+  double p[2 * KT];
+  R w;
+};
+template <class R, int KT>
+__device__ __forceinline__ LrFetched<R, KT> lr_fetch(const LrArgs<R> &l, const LrPlace &pl, int K) {
+  LrFetched<R, KT> f;
+  const bool two = blockDim.x > kBlock;
 #pragma unroll
-  for (int j = 0; j < kLrPre; ++j) {
-    const int b = lane + j * kWave;
-    pre[j] = wave < 2 * K && b < nparts ? part[(size_t)wave * nparts + b] : 0.0;
+  for (int j = 0; j < 2 * KT; ++j) {
+    const int jj = j < KT ? j : j - KT;  // two: value jj of the half, partials t (j < KT) and t + kBlock
+    const int q = two ? pl.half * K + jj : j, b = pl.tid + (two && j >= KT ? kBlock : 0);
+    f.p[j] = (two ? jj < K : j < 2 * K) && b < l.blocks ? l.part_in[(size_t)q * l.blocks + b] : 0.0;
   }
+  f.w = l.w[(int)threadIdx.x < 2 * K ? threadIdx.x >> 1 : 0];
+  return f;
 }
-template <class R>
-__device__ __forceinline__ void lr_reduce(const double *part, int nparts, int K, const R *w,
-                                          const double (&pre)[kLrPre], double *g) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, nw = blockDim.x / kWave;
-  for (int q = wave; q < 2 * K; q += nw) {
-    double t = 0.0;
-    if (q == wave) {
+template <class R, int KT>
+__device__ __forceinline__ void lr_reduce(const LrFetched<R, KT> &f, const LrPlace &pl, int K, double *g) {
+  constexpr int NV = lr_pow2(2 * KT), NH = lr_pow2(KT);
+  __shared__ double red[kLrBlockWaves][NV + NH];
+  const int lane = threadIdx.x % kWave;
+  if (blockDim.x > kBlock) {
+    double v[NH];
 #pragma unroll
-      for (int j = 0; j < kLrPre; ++j) t += pre[j];
-    }
-#pragma unroll 4
-    for (int b = lane + (q == wave ? kLrPre * kWave : 0); b < nparts; b += kWave) t += part[(size_t)q * nparts + b];
-    t = wave_sum(t);
-    if (lane == 0) g[q] = t * (double)w[q >> 1];
+    for (int j = 0; j < NH; ++j) v[j] = j < KT ? f.p[j < KT ? j : 0] + f.p[j < KT ? KT + j : 0] : 0.0;
+    const double t = wave_reduce<double, NH>(v, lane);
+    const int slot = wave_slot<NH>(lane);
+    if (slot < K) red[pl.wave][pl.half * K + slot] = t;
+  } else {
+    double v[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[j] = j < 2 * KT ? f.p[j < 2 * KT ? j : 0] + 0.0 : 0.0;
+    const double t = wave_reduce<double, NV>(v, lane);
+    red[pl.wave][wave_slot<NV>(lane)] = t;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < 2 * K) {
+    double t = red[0][threadIdx.x];
+#pragma unroll
+    for (int q = 1; q < kLrBlockWaves; ++q) t += red[q][threadIdx.x];
+    g[threadIdx.x] = t * (double)f.w;
   }
   __syncthreads();
 }
-
-template <class R> struct LrArgs {
-  const R *XT;  // [K][ldv], zero past N
-  const R *w;   // [K]
-  int K;
-  const double *part_in;  // [2K][nparts]
-  int nparts;
-  double *part_out;       // [2K][gridDim.x]
-};
 
 template <class R, int KT, bool EXACT>
 __device__ __forceinline__ void lr_load_row(const LrArgs<R> &l, int K, long ldv, long i, R (&x)[KT]) {
@@ -931,28 +971,29 @@ __device__ __forceinline__ void lr_accumulate(const R (&x)[KT], int K, R c, R s,
 }
 
 template <class R, int KT, bool EXACT>
-__global__ __launch_bounds__((kLrThreads<R, KT>)) void lowrank_gram_kernel(const LrArgs<R> l, long N, const R *cs, long ldv) {
+__global__ __launch_bounds__(kLrThreads) void lowrank_gram_kernel(const LrArgs<R> l, long N, const R *cs, long ldv) {
   const int K = EXACT ? KT : l.K;
+  const LrPlace pl(l.blocks);
   double acc[2 * KT] = {};
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) {
+  for (long i = pl.first(N); i < N; i += (long)l.blocks * kBlock) {
     R x[KT];
     lr_load_row<R, KT, EXACT>(l, K, ldv, i, x);
     lr_accumulate<R, KT, EXACT>(x, K, cs[i], cs[ldv + i], acc);
   }
-  lr_write_partials<R, KT>(acc, K, l.part_out);
+  lr_write_partials<KT>(pl, acc, K, l.blocks, l.part_out);
 }
 
 template <class R, int KIND, int KT, bool EXACT>
-__global__ __launch_bounds__((kLrThreads<R, KT>)) void lowrank_stage_kernel(const LrArgs<R> l, const Vecs<R> v) {
+__global__ __launch_bounds__(kLrThreads) void lowrank_stage_kernel(const LrArgs<R> l, const Vecs<R> v) {
   constexpr bool NEXT = KIND >= 2 && KIND < 7;  // also the partials of the vector this stage writes
   __shared__ double gs[2 * KT];
   const int K = EXACT ? KT : l.K;
+  const LrPlace pl(l.blocks);
   // everything the first row needs is in flight before the state check and
   // the reduction of G (rows past N re-read row N - 1, never used)
-  const long stride = (long)gridDim.x * blockDim.x;
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  double pre[kLrPre];
-  lr_fetch(l.part_in, l.nparts, K, pre);
+  const long stride = (long)l.blocks * kBlock;
+  long i = pl.first(v.N);
+  const LrFetched<R, KT> fetched = lr_fetch<R, KT>(l, pl, K);
   R x[KT];
   const long i0 = i < v.N ? i : v.N - 1;
   lr_load_row<R, KT, EXACT>(l, K, v.ldv, i0, x);
@@ -961,10 +1002,18 @@ __global__ __launch_bounds__((kLrThreads<R, KT>)) void lowrank_stage_kernel(cons
   if constexpr (KIND >= 2) {
     if (v.check_state && (!v.st->active || v.st->commit_pending)) return;
   }
-  lr_reduce<R>(l.part_in, l.nparts, K, l.w, pre, gs);
+  lr_reduce<R, KT>(fetched, pl, K, gs);
   double acc[2 * KT] = {};
   double sq = 0.0;
   while (i < v.N) {
+    // the next row's operands are in flight while this row is computed
+    R xn[KT];
+    RowOps<R, KIND> opsn;
+    const bool more = i + stride < v.N;
+    if (more) {
+      lr_load_row<R, KT, EXACT>(l, K, v.ldv, i + stride, xn);
+      opsn = row_load<R, KIND>(v, i + stride);
+    }
     asm volatile("" ::: "memory");  // G is re-read from LDS for every row: in registers it would cost 4K of them
     double C = 0, S = 0;
 #pragma unroll
@@ -977,23 +1026,22 @@ __global__ __launch_bounds__((kLrThreads<R, KT>)) void lowrank_stage_kernel(cons
     sq += row_finish<R, KIND>(v, i, ops, (R)C, (R)S, &c, &s);
     if constexpr (NEXT) lr_accumulate<R, KT, EXACT>(x, K, c, s, acc);
     i += stride;
-    if (i < v.N) {
-      lr_load_row<R, KT, EXACT>(l, K, v.ldv, i, x);
-      ops = row_load<R, KIND>(v, i);
+    if (more) {
+#pragma unroll
+      for (int m = 0; m < KT; ++m) x[m] = xn[m];
+      ops = opsn;
     }
   }
   if constexpr (KIND == 7) {
-    __shared__ double errsq[kLrThreads<R, KT> / kWave];
-    const double t = wave_sum(sq);
-    if (threadIdx.x % kWave == 0) errsq[threadIdx.x / kWave] = t;
+    __shared__ double errsq[2][kBlock];
+    errsq[pl.half][pl.tid] = sq;
     __syncthreads();
-    if (threadIdx.x == 0) {
-      double tot = errsq[0];
-      for (int q = 1; q < (int)blockDim.x / kWave; ++q) tot += errsq[q];
-      v.err_part[blockIdx.x] = tot;
+    if (pl.wave == 0) {
+      const double tot = block_tree(errsq[pl.half]);
+      if (pl.tid == 0 && pl.live) v.err_part[pl.blk] = tot;
     }
   }
-  if constexpr (NEXT) lr_write_partials<R, KT>(acc, K, l.part_out);
+  if constexpr (NEXT) lr_write_partials<KT>(pl, acc, K, l.blocks, l.part_out);
 }
 
 // r = sqrt((X/N)^2 + (Y/N)^2) in the working precision (kuramoto.cu:220:
@@ -1193,16 +1241,17 @@ __device__ __forceinline__ void stage2_vector(const EmitArgs<R> &a, long i, R y,
   a.cs_out[a.ldv + i] = s;
 }
 
-// n output rows of one dense-output interval: te(q) the q-th output time,
-// put(q, value) keeps this thread's value, part(q) the row's partial sums of
-// this workgroup.  Four rows at a time: their cos / sin, then one wave sums
-// each row (block_tree), so a group of rows costs two barriers and one chain
-// of latencies (one row at a time: 12 rows of N = 10^4 took 21 us).
+// n output rows of one dense-output interval, for each kBlock threads of a
+// workgroup: te(q) the q-th output time, put(q, value) keeps this thread's
+// value, part(q, sums) the row's partial sums of these threads.  Four rows at
+// a time: their cos / sin, then one wave sums each row (block_tree), so a
+// group of rows costs two barriers and one chain of latencies (one row at a
+// time: 12 rows of N = 10^4 took 21 us).
 constexpr int kEmitRows = kBlock / kWave;
 template <class R, class TE, class PUT, class PART>
 __device__ __forceinline__ void emit_rows(int n, bool valid, const R Q[4], R yl, R tl, R hh,
                                           double (&sh)[kEmitRows][2][kBlock], TE te, PUT put, PART part) {
-  const int tid = threadIdx.x, wave = tid / kWave;
+  const int tid = threadIdx.x % kBlock, wave = tid / kWave;
   for (int q0 = 0; q0 < n; q0 += kEmitRows) {
     const int m = n - q0 < kEmitRows ? n - q0 : kEmitRows;
 #pragma unroll
@@ -1221,7 +1270,7 @@ __device__ __forceinline__ void emit_rows(int n, bool valid, const R Q[4], R yl,
     __syncthreads();
     if (wave < m) {
       const double bc = block_tree(sh[wave][0]), bs = block_tree(sh[wave][1]);
-      if (tid % kWave == 0) *part(q0 + wave) = make_double2(bc, bs);
+      if (tid % kWave == 0) part(q0 + wave, make_double2(bc, bs));
     }
     __syncthreads();
   }
@@ -1258,8 +1307,8 @@ template <class R> __device__ __forceinline__ bool emit_commit(const EmitArgs<R>
         [&](int q, R val) {
           if (a.ring) a.ring[(size_t)(slot0 + q) * a.ldv + i] = val;
         },
-        [&](int q) {
-          return reinterpret_cast<double2 *>(a.ord_part) + (size_t)(slot0 + q) * gridDim.x + blockIdx.x;
+        [&](int q, double2 sums) {
+          reinterpret_cast<double2 *>(a.ord_part)[(size_t)(slot0 + q) * gridDim.x + blockIdx.x] = sums;
         });
   }
   if (mode == JOB_COMMIT && valid) {
@@ -1277,74 +1326,62 @@ __global__ __launch_bounds__(kBlock) void emit_commit_kernel(const EmitArgs<R> a
   (void)emit_commit<R>(a, (long)blockIdx.x * kBlock + threadIdx.x, c, s);
 }
 
-// emit_commit_kernel for the low-rank path, on its grid (threads stride over
-// the rows), with the partials of X^T (cos, sin) of the stage-2 vector it
-// writes.  Output rows four at a time: each wave's 8 sums by wave_reduce,
-// then the waves in order.
+// emit_commit_kernel for the low-rank path, on its blocks, with the partials
+// of X^T (cos, sin) of the stage-2 vector it writes.  nblk: order partials of
+// an output row (one per kBlock rows).
 template <class R, int KT, bool EXACT>
-__global__ __launch_bounds__((kLrThreads<R, KT>)) void lowrank_emit_kernel(const EmitArgs<R> a, const LrArgs<R> l) {
+__global__ __launch_bounds__(kLrThreads) void lowrank_emit_kernel(const EmitArgs<R> a, const LrArgs<R> l, int nblk) {
   const State<R> *st = a.st;
   const int mode = st->job_mode;
   if (mode == JOB_NONE) return;
-  constexpr int ER = 4;
-  __shared__ double red[kLrThreads<R, KT> / kWave][2 * ER];
+  __shared__ double sh[2][kEmitRows][2][kBlock];
   const int K = EXACT ? KT : l.K;
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, nw = blockDim.x / kWave;
-  const long first = (long)blockIdx.x * blockDim.x + tid, stride = (long)gridDim.x * blockDim.x;
+  const LrPlace pl(l.blocks);
+  const long stride = (long)l.blocks * kBlock, first = pl.first(a.N);
   const R h = st->h;
   const int n_emit = mode == JOB_STAGE2 ? 0 : st->job_n, slot0 = st->job_slot, lo = st->job_lo;
   const R tl = st->t_last, hh = st->t - tl;
-  for (int q0 = 0; q0 < n_emit; q0 += ER) {
-    double v[2 * ER] = {};
-    for (long i = first; i < a.N; i += stride) {
-      R kv[7], Q[4];
-#pragma unroll
-      for (int j = 0; j < 7; ++j) kv[j] = a.k[j][i];
-      dense_coeffs<R>(kv, Q);
-      const R yl = a.y[i];
-#pragma unroll
-      for (int r = 0; r < ER; ++r) {
-        if (q0 + r >= n_emit) break;
-        const R val = dense_value<R>(Q, yl, hh, (a.t_eval[lo + q0 + r] - tl) / hh);
-        if (a.ring) a.ring[(size_t)(slot0 + q0 + r) * a.ldv + i] = val;
-        R c, s;
-        rsincos<R>(val, c, s);
-        v[2 * r] += (double)c;
-        v[2 * r + 1] += (double)s;
-      }
-    }
-    const double t = wave_reduce<double, 2 * ER>(v, lane);
-    red[wave][wave_slot<2 * ER>(lane)] = t;
-    __syncthreads();
-    if (tid < 2 * ER && q0 + tid / 2 < n_emit) {
-      double sum = red[0][tid];
-      for (int w = 1; w < nw; ++w) sum += red[w][tid];
-      a.ord_part[((size_t)(slot0 + q0 + tid / 2) * gridDim.x + blockIdx.x) * 2 + tid % 2] = sum;
-    }
-    __syncthreads();
-  }
-  if (mode == JOB_EMIT) return;
   double acc[2 * KT] = {};
-  for (long i = first; i < a.N; i += stride) {
-    R x[KT];
-    lr_load_row<R, KT, EXACT>(l, K, a.ldv, i, x);
-    R y = a.y[i], k1 = a.k[0][i];
+  // the first half's block reaches as far as the second's: the same passes for both
+  for (long p = 0; (long)blockIdx.x * kBlock + p * stride < a.N; ++p) {
+    const long i = first + p * stride;
+    const bool valid = i < a.N;
+    R x[KT], y = 0, k1 = 0, yn = 0, k7 = 0;
+    if (valid) {
+      lr_load_row<R, KT, EXACT>(l, K, a.ldv, i, x);
+      y = a.y[i], k1 = a.k[0][i], yn = a.ynew[i], k7 = a.k[6][i];
+    }
+    if (n_emit > 0) {
+      R Q[4] = {0, 0, 0, 0};
+      if (valid) {
+        R kv[7];
+        kv[0] = k1, kv[6] = k7;
+#pragma unroll
+        for (int j = 1; j < 6; ++j) kv[j] = a.k[j][i];
+        dense_coeffs<R>(kv, Q);
+      }
+      const long blk = pl.blk + p * l.blocks;
+      emit_rows<R>(
+          n_emit, valid, Q, y, tl, hh, sh[pl.half], [&](int q) { return a.t_eval[lo + q]; },
+          [&](int q, R val) {
+            if (a.ring) a.ring[(size_t)(slot0 + q) * a.ldv + i] = val;
+          },
+          [&](int q, double2 sums) {
+            if (pl.live && blk < nblk) reinterpret_cast<double2 *>(a.ord_part)[(size_t)(slot0 + q) * nblk + blk] = sums;
+          });
+    }
+    if (mode == JOB_EMIT || !valid) continue;
     if (mode == JOB_COMMIT) {
       // commit (dp45.cu:123-125, FSAL copy :160)
       a.ylast[i] = y;
-      y = a.ynew[i];
-      k1 = a.k[6][i];
-      a.y[i] = y;
-      a.k[0][i] = k1;
+      a.y[i] = y = yn;
+      a.k[0][i] = k1 = k7;
     }
-    const R yt = rfma<R>(k1 * (R)tab::A[0][0], h, y);
     R c, s;
-    rsincos<R>(yt, c, s);
-    a.cs_out[i] = c;
-    a.cs_out[a.ldv + i] = s;
+    stage2_vector<R>(a, i, y, k1, h, c, s);
     lr_accumulate<R, KT, EXACT>(x, K, c, s, acc);
   }
-  lr_write_partials<R, KT>(acc, K, l.part_out);
+  if (mode != JOB_EMIT) lr_write_partials<KT>(pl, acc, K, l.blocks, l.part_out);
 }
 
 // ---------------------------------------------------------------------
