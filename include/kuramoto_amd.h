@@ -231,14 +231,15 @@ int kmt_bandwidth_probe(int device, size_t bytes, int reps, double *copy_gbps, d
  * average ms of each variant (the faster ring form for one workgroup per
  * group), index 4*r + 2*nt + balanced with r = 0, 1, 2 for 4, 8, 16 rows.
  * Every row is summed in the same order in every variant; the error norm's
- * partial sums follow the variant's workgroups (the ring groups them as the
- * loop without it does), so its last bits (and h's) can differ between
+ * partial sums follow the pinned variant's workgroups (the ring groups them as
+ * the loop without it does), so its last bits (and h's) can differ between
  * variants.  Without this call a fixed choice is used (a matrix of up to
  * 256 MB: plain loads, 4 rows, 8 for N < 4096 and for 16-bit entries with
  * FP64 state; a larger one: non-temporal loads, 8 rows, 16 for 16-bit
- * entries with FP64 state or N >= 50000; the chunk ring for the working precision, and for 16-bit entries
- * of up to 256 MB with FP32 state), so that every context and process gives
- * the same bits.
+ * entries with FP64 state or N >= 50000; the chunk ring for the working
+ * precision, and for 16-bit entries of up to 256 MB with FP32 state), and the
+ * error norm is grouped by 8 rows (16 for 16-bit entries; 4 from N = 4096 on
+ * up to 128 MB), so that every context and process gives the same bits.
  * Calling it (mid-run, or in only one of two contexts) therefore breaks
  * bit-exact restart against contexts that use the fixed choice.  KMT_ADJ_SYM has one
  * form and is not tuned.  No reference counterpart (cuBLAS chooses its own

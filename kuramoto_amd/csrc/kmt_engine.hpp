@@ -227,10 +227,12 @@ template <class R> struct Engine : EngineBase {
     return KMT_OK;
   }
   // The stage-7 error partials are summed per workgroup, so their grouping,
-  // and with it the last bits of the error norm and of h, follows the
-  // variant.  kmt_begin therefore picks it by a fixed rule, not by timing,
+  // and with it the last bits of the error norm and of h, follows the rows of
+  // stage 7's variant.  Those are a rule of their own (error_rows) that says
+  // nothing about speed, and every choice is by a fixed rule, not by timing,
   // so that runs and restarts of one problem give the same bits in every
-  // context and process.
+  // context and process.  The other stages write no partials and sum every
+  // row in the same order in every variant:
   //  * A matrix that fits the 256 MB Infinity Cache is read from it by every
   //    stage after the first, so its loads are plain (a non-temporal load
   //    does not keep the line: FP64 N=5000, 200 MB, 34.8 -> 30.6 us; FP32
@@ -240,7 +242,7 @@ template <class R> struct Engine : EngineBase {
   //    (17.8 against 18.2 us with 8 rows, 20.9 with 16).  With FP64 vectors
   //    and 16-bit entries 8 rows: the vectors' bytes are then no more than the
   //    entries' (BF16 N=8000: 26.1 us against 30.7 with 4 rows).  Smaller N
-  //    keep 8 rows, the grouping of the FP64 register-rebuild kernel.
+  //    keep 8 rows.
   //  * A larger one takes 8 rows with non-temporal loads, 16 rows with 16-bit
   //    entries (each (cos, sin) chunk is reused for every row of the group:
   //    FP64 state, BF16, N=50000: 0.752 against 0.812 ms with 8 rows; FP32
@@ -262,6 +264,15 @@ template <class R> struct Engine : EngineBase {
     bal_grid = 0;
     tuned = 1;
     drop_graphs();
+  }
+
+  // Rows per error partial.  16-bit entries: 16; the working precision: 8 (the
+  // grouping of the FP64 register-rebuild kernel, whose runs are the dense
+  // ones' bit for bit); 4 for matrices of 4096 rows up to 128 MB.
+  int error_rows() const {
+    if (pinned) return tune_rows;
+    if (N >= 4096 && (double)N * (double)N * (double)elem_bytes(storage) <= 128e6) return 4;
+    return elem_bytes(storage) == 2 ? 16 : 8;
   }
 
   // Every entry point that launches the dense kernel uses the rule's choice:
@@ -883,7 +894,7 @@ template <class R> struct Engine : EngineBase {
     if (tune_bal) {
       if (bal_grid <= 0) bal_grid = balanced_grid<S, ROWS, NT>();
       stage_kernel<R, S, ROWS, KIND, NT, true><<<(unsigned)bal_grid, kBlock, 0, stream>>>(a);
-    } else if (tune_ring) {
+    } else if (tune_ring && (pinned || ROWS < 16 || sizeof(S) > 2)) {
       const unsigned grid = (unsigned)((N + ROWS - 1) / ROWS);
       stage_ring_kernel<R, S, ROWS, KIND, NT><<<grid, kBlock, 0, stream>>>(a);
     } else {
@@ -898,7 +909,7 @@ template <class R> struct Engine : EngineBase {
     a.lda = lda;
     a.mscale = (R)mscale_;
     a.v = v;
-    switch (tune_rows * 2 + (tune_nt ? 1 : 0)) {
+    switch ((KIND == 7 ? error_rows() : tune_rows) * 2 + (tune_nt ? 1 : 0)) {
       case 8: launch_dense_variant<S, KIND, 4, false>(a); break;
       case 9: launch_dense_variant<S, KIND, 4, true>(a); break;
       case 16: launch_dense_variant<S, KIND, 8, false>(a); break;
@@ -1091,7 +1102,7 @@ template <class R> struct Engine : EngineBase {
     if (factored) return lr_fused() ? lr_blocks : (int)((N + kBlock - 1) / kBlock);
     if (sym()) return (int)sym_nb;
     if (tune_bal) return bal_grid;
-    return (int)((N + tune_rows - 1) / tune_rows);
+    return (int)((N + error_rows() - 1) / error_rows());
   }
 
   // Autotuner of the dense stage kernel: rows per workgroup {4, 8, 16} x
