@@ -312,8 +312,9 @@ int kmt_batch_get_instance(kmt_batch *batch, int b, float *theta, double *state8
 int kmt_batch_autotune(kmt_batch *batch, int reps, int *variant, int *split_k, double *best_ms);
 int kmt_batch_tune_table(kmt_batch *batch, double *ms96);
 /* pin the shared product's workgroup variant and split-K instead of the
- * autotuner's choice (without either, kmt_batch_begin takes variant 3 and the
- * split by a rule on N and B) */
+ * autotuner's choice.  Without either, kmt_batch_begin takes variant 3 and
+ * split 8 for adaptive steps, and for a fixed step the split by a rule on N
+ * and B: the split is the order of FP32 sums, which step sizes follow from. */
 int kmt_batch_select_tile(kmt_batch *batch, int variant, int split_k);
 /* shared mode: once finished instances leave the active ones fitting in
  * fewer 32-row MFMA tiles, kmt_batch_advance renumbers the active instances'

@@ -1132,29 +1132,36 @@ struct kmt_batch {
     else if (mt_act == 3) gemm_mt<T, 3>();
     else gemm_mt<T, 4>();
   }
-  // Split-K without the caller's choice: the grid is (row blocks x split)
-  // workgroups of 256 rows, one per CU at a time, so a split costs whole
-  // rounds of its slab's chunks, and its partials are written here and read
-  // back by the epilogue.  Of the splits 1..16, the one with the smallest
-  // rounds (slab chunks t_chunk + 3 us) + partials at 5 TB/s, with t_chunk =
-  // 0.6 us + 0.34 us per 32 rows of hi + lo vectors (half without lo) as
-  // measured at B = 64 and 32, N = 20000.  There it picks 3 (240 workgroups,
-  // one round) instead of the former 8 (640, two and a half): 206 against 234
-  // us per product and 31 against 84 MB of partials per stage; at N = 8000 it
-  // keeps 8 (256 workgroups).  Chosen once per run for the whole batch, so
-  // that compacting the rows of finished instances does not change the sums.
+  // Split-K without the caller's choice.  Adaptive steps: 8, whatever N and B:
+  // the split is the order of FP32 sums, and a last bit of a coupling is
+  // another sequence of steps a few attempts later (another split changed the
+  // accepted counts of 64 Cauchy networks of N = 2000 within 12 attempts).
+  // A fixed step has no sequence to keep, and takes the cheapest: the grid is
+  // (row blocks x split) workgroups of 256 rows, one per CU at a time, so a
+  // split costs whole rounds of its slab's chunks, and its partials are
+  // written here and read back by the epilogue.  Of the splits 1..16, the one
+  // with the smallest rounds (slab chunks t_chunk + 3 us) + partials at 5 TB/s,
+  // with t_chunk = 0.6 us + 0.34 us per 32 rows of hi + lo vectors (half
+  // without lo) as measured at B = 64 and 32, N = 20000, and rounds of 256
+  // workgroups whatever the card's partition, so that N and B alone decide the
+  // order.  At B = 64, N = 20000 it picks 3 (240 workgroups, one round) instead
+  // of 8 (640, two and a half): 206 against 234 us per product and 31 against
+  // 84 MB of partials per stage; at N = 8000 it keeps 8 (256 workgroups).
+  // Chosen once per run for the whole batch, so that compacting the rows of
+  // finished instances does not change the sums.
   void default_split() {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) cus = 1;
+    tile_var = 3;
+    ksplit = 8;
+    if (!fixed) return;
+    constexpr long kRound = 256;
     const long nkc = lda_shared / kKC, nrb = rows_shared / 256;
     const double t_chunk = 0.6e-6 + 0.34e-6 * mt * (lo ? 1.0 : 0.5);
     double best = 1e30;
     for (int c = 1; c <= 16; ++c) {
-      const long slab = (nkc + c - 1) / c, rounds = (nrb * c + cus - 1) / cus;
+      const long slab = (nkc + c - 1) / c, rounds = (nrb * c + kRound - 1) / kRound;
       const double t = rounds * (slab * t_chunk + 3e-6) + 2.0 * c * mpad * (double)ldn * sizeof(float) / 5e12;
       if (t < best) best = t, ksplit = c;
     }
-    tile_var = 3;
   }
   void coupling(int check) {
     if (shared) {
