@@ -859,10 +859,12 @@ struct kmt_batch {
   float *r_ring = nullptr, *t_eval = nullptr;
   BInst *inst = nullptr;
   std::vector<BInst> host_inst;
-  // host_inst of a run equals the device's records (nothing launched since
-  // they were fetched) up to the rings' drained counts; inst_dirty: those are
-  // not written back yet.  r_host: the rings as of then (r_valid).
-  bool inst_fresh = false, inst_dirty = false, r_valid = false;
+  // inst_fresh: host_inst holds the records (nothing launched since they were
+  // fetched; before the first run they exist here only), and what the host
+  // changed in them since - drained counts, an instance's or a factor's new
+  // values - is in the device's once flush() has written them back
+  // (inst_dirty).  r_host: the rings as of then (r_valid).
+  bool inst_fresh = true, inst_dirty = false, r_valid = false;
   float *r_host = nullptr;  // pinned, B x ring_cap
   void *A = nullptr;
   size_t A_bytes = 0;
@@ -968,13 +970,14 @@ struct kmt_batch {
 
   int set_instance(int b, const float *omega, const float *theta, double c1, double t0, double h0) {
     if (b < 0 || b >= B) return kmt_fail(KMT_ERR_ARG, "instance %d out of range", b);
-    KMT_TRY(flush());  // host_inst is changed below
+    KMT_TRY(fetch());  // host_inst is changed below
     HIP_TRY(hipMemcpyAsync(om + (size_t)b * ldn, omega, sizeof(float) * Nb[b], hipMemcpyHostToDevice, stream));
     HIP_TRY(hipMemcpyAsync(y + (size_t)b * ldn, theta, sizeof(float) * Nb[b], hipMemcpyHostToDevice, stream));
     HIP_TRY(hipStreamSynchronize(stream));
     host_inst[b].c1 = (float)c1;
     host_inst[b].t = (float)t0;
     host_inst[b].h = (float)h0;
+    inst_dirty = true;
     begun = 0;
     return KMT_OK;
   }
@@ -1014,7 +1017,7 @@ struct kmt_batch {
   // dense adjacency of instance b (or the shared one, b = -1) from a factor
   int set_factor(int b, const float *Xh, const float *wh, int K) {
     if (shared ? b != -1 : (b < 0 || b >= B)) return kmt_fail(KMT_ERR_ARG, "instance %d: use -1 for the shared adjacency", b);
-    KMT_TRY(flush());  // host_inst is changed below
+    KMT_TRY(fetch());  // host_inst is changed below
     KMT_TRY(ensure_A());
     const long N = shared ? Nmax : Nb[b];
     double mx = 0;
@@ -1060,6 +1063,7 @@ struct kmt_batch {
     if (shared)
       for (int q = 0; q < B; ++q) { mscale[q] = (float)sc; host_inst[q].mscale = (float)sc; }
     else { mscale[b] = (float)sc; host_inst[b].mscale = (float)sc; }
+    inst_dirty = true;
     drop_graphs();
     return KMT_OK;
   }
@@ -1364,7 +1368,7 @@ struct kmt_batch {
     if (inst_fresh) return KMT_OK;
     HIP_TRY(hipMemcpyAsync(host_inst.data(), inst, sizeof(BInst) * B, hipMemcpyDeviceToHost, stream));
     HIP_TRY(hipStreamSynchronize(stream));
-    inst_fresh = begun;
+    inst_fresh = true;
     return KMT_OK;
   }
   // before launches that change the records
@@ -1551,7 +1555,9 @@ struct kmt_batch {
       // operands and then run at higher clocks, which makes every candidate
       // look faster than it is inside a run.  (After kmt_batch_begin the
       // buffers hold the current stage's vectors; begin rewrites them.)
+      KMT_TRY(fetch());
       HIP_TRY(hipMemcpyAsync(inst, host_inst.data(), sizeof(BInst) * B, hipMemcpyHostToDevice, stream));
+      inst_dirty = false;
       dim3 g2((unsigned)nblk, (unsigned)B);
       if (storage == KMT_ADJ_F16) bsincos_kernel<f16_t><<<g2, kBlock, 0, stream>>>(y, inst, ldn, cs[1], vt_out(), 1);
       else bsincos_kernel<bf16_t><<<g2, kBlock, 0, stream>>>(y, inst, ldn, cs[1], vt_out(), 1);
