@@ -276,10 +276,13 @@ template <class R> struct Engine : EngineBase {
   }
 
   // Every entry point that launches the dense kernel uses the rule's choice:
-  // a right-hand side evaluated before any run too (it used to take 8 rows
-  // without the ring whatever the storage: FP64 state, BF16, N=50000 0.802 ms
-  // against 0.757 with 16 rows).  Rows are summed in the same order in every
-  // variant.  No HIP call when there is nothing to drop: safe under capture.
+  // a right-hand side evaluated before any run too (with 8 rows and no ring
+  // whatever the storage, FP64 state, BF16, N=50000 took 0.802 ms against
+  // 0.757 with 16 rows), and a run that comes to the dense form between
+  // advances (from a factor, or with another storage), so that an evaluation
+  // in between does not change the run.  Rows are summed in the same order in
+  // every variant.  No HIP call when there is nothing to drop: safe under
+  // capture.
   void ensure_variant() {
     if (!tuned && !factored && !sym()) default_variant();
   }
@@ -1244,6 +1247,7 @@ template <class R> struct Engine : EngineBase {
   }
   // n attempts of the run
   int launch_attempts(int n) {
+    ensure_variant();
     if (small_path()) {
       SmallArgs<R> a;
       a.A = (const R *)A;
@@ -1447,6 +1451,7 @@ template <class R> struct Engine : EngineBase {
       return KMT_OK;
     }
     if (rows && n > 0) KMT_TRY(drain_rows(rows, ring, sizeof(R) * ldv, sizeof(R) * N, n));
+    if (cpl && n > 0) ensure_variant();
     for (int q = 0; cpl && q < n; ++q) {
       sincos_kernel<R><<<(unsigned)((N + kBlock - 1) / kBlock), kBlock, 0, stream>>>(ring + (size_t)q * ldv, N, ldv, cs_scr);
       Vecs<R> v = vecs(cs_scr, nullptr, 0);
@@ -1552,6 +1557,7 @@ template <class R> struct Engine : EngineBase {
     KMT_TRY(fetch_state());
     if (attempts > shadow.times_cap - shadow.times_count)
       return fail(KMT_ERR_ARG, "attempts exceed the accepted-step log capacity; drain kmt_read_times first");
+    ensure_variant();
     std::vector<std::pair<hipEvent_t, hipEvent_t>> pairs_all(6 * attempts);
     for (auto &p : pairs_all) {
       HIP_TRY(hipEventCreate(&p.first));
