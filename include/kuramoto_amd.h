@@ -211,7 +211,10 @@ int kmt_eval(kmt_ctx *ctx, double t_eval, void *theta);
 int kmt_time_stage_kernel(kmt_ctx *ctx, int reps, double *avg_ms);
 /* Time `attempts` step attempts on the library's stream with HIP events;
  * reports wall ms for the whole region and the average ms of the stage
- * kernel launches inside it (events around each stage launch). */
+ * kernel launches inside it (events around each stage launch).  A dense
+ * network small enough for whole attempts in one workgroup (working
+ * precision, N <= 256 FP32 or 128 FP64) has no stage launches: its region is
+ * what kmt_advance runs, and the stage average a sixth of it per attempt. */
 int kmt_time_attempts(kmt_ctx *ctx, int attempts, double *region_ms, double *stage_avg_ms, kmt_status *st);
 
 /* Measured bandwidth ceiling of the device: a plain 16-byte copy kernel
@@ -242,11 +245,14 @@ int kmt_bandwidth_probe(int device, size_t bytes, int reps, double *copy_gbps, d
  * up to 128 MB), so that every context and process gives the same bits.
  * Calling it (mid-run, or in only one of two contexts) therefore breaks
  * bit-exact restart against contexts that use the fixed choice.  KMT_ADJ_SYM has one
- * form and is not tuned.  No reference counterpart (cuBLAS chooses its own
+ * form and is not tuned; the attempts of a network of N <= 256 (FP32) or 128
+ * (FP64) in the working precision stay in one workgroup, with the fixed
+ * choice's bits, and the tuned variant serves its right-hand sides.  No reference counterpart (cuBLAS chooses its own
  * gemv kernel). */
 int kmt_autotune(kmt_ctx *ctx, int reps, double *variant_ms);
 /* Pin the dense stage-kernel variant instead of the autotuner's choice:
- * rows per group 4, 8 or 16; variant_flags as kmt_layout reports them. */
+ * rows per group 4, 8 or 16; variant_flags as kmt_layout reports them.
+ * Attempts of small networks then take it too, instead of one workgroup. */
 int kmt_select_variant(kmt_ctx *ctx, int rows_per_block, int variant_flags);
 
 /* Sizes the library chose (for roofline bookkeeping): padded row stride of

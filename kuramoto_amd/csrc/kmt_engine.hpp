@@ -130,7 +130,7 @@ template <class R> struct Engine : EngineBase {
   hipGraphExec_t g1 = nullptr, g8 = nullptr;
   bool graphs_valid = false;
   int tune_rows = 8, tune_nt = 1, tune_bal = 0, tune_ring = 0, tuned = 0;
-  int pinned = 0;  // variant chosen by the caller (kmt_select_variant, kmt_autotune)
+  int pinned = 0;  // attempts follow a variant chosen by the caller (kmt_select_variant) or timed (kmt_autotune)
   double tune_ms[12] = {0};
   int bal_grid = 0;  // workgroups of the balanced variant (one resident round)
   R t0_ = 0, h0_ = 0;
@@ -1169,7 +1169,10 @@ template <class R> struct Engine : EngineBase {
     tune_bal = best_bal;
     tune_ring = best_ring;
     bal_grid = best_grid;
-    tuned = pinned = 1;
+    tuned = 1;
+    // the timed form is for right-hand sides only where attempts have a
+    // faster one (N = 200 FP32: 16 us against 32 per attempt)
+    pinned = !small_size();
     drop_graphs();
     return KMT_OK;
   }
@@ -1232,10 +1235,9 @@ template <class R> struct Engine : EngineBase {
 
   // Small dense networks in the working precision: whole attempts in one
   // workgroup, as far as its registers hold the matrix.  A caller's own
-  // choice of stage variant keeps the launched kernels.
-  bool small_path() const {
-    return !factored && A && storage == KMT_ADJ_NATIVE && !pinned && N <= kSmallMaxN<R>;
-  }
+  // choice of stage variant (kmt_select_variant) keeps the launched kernels.
+  bool small_size() const { return !factored && A && storage == KMT_ADJ_NATIVE && N <= kSmallMaxN<R>; }
+  bool small_path() const { return small_size() && !pinned; }
   template <int G> void launch_small(const SmallArgs<R> &a, int n) {
     if constexpr (G < kSmallMaxGroups<R>) {
       if (N > (long)G * 8 * kSmallWaves) {
@@ -1558,7 +1560,8 @@ template <class R> struct Engine : EngineBase {
     if (attempts > shadow.times_cap - shadow.times_count)
       return fail(KMT_ERR_ARG, "attempts exceed the accepted-step log capacity; drain kmt_read_times first");
     ensure_variant();
-    std::vector<std::pair<hipEvent_t, hipEvent_t>> pairs_all(6 * attempts);
+    const bool launches = !small_path();  // the one-workgroup form has no stage launches to time
+    std::vector<std::pair<hipEvent_t, hipEvent_t>> pairs_all(launches ? 6 * attempts : 0);
     for (auto &p : pairs_all) {
       HIP_TRY(hipEventCreate(&p.first));
       HIP_TRY(hipEventCreate(&p.second));
@@ -1568,10 +1571,14 @@ template <class R> struct Engine : EngineBase {
     HIP_TRY(hipEventCreate(&r1));
     std::vector<std::pair<hipEvent_t, hipEvent_t>> work = pairs_all;
     KMT_TRY(flush_state());
-    launch_prepare();
+    if (launches) launch_prepare();
     HIP_TRY(hipEventRecord(r0, stream));
-    for (int a = 0; a < attempts; ++a) launch_attempt(&work);
-    launch_finalize();
+    if (launches) {
+      for (int a = 0; a < attempts; ++a) launch_attempt(&work);
+      launch_finalize();
+    } else {
+      KMT_TRY(launch_attempts(attempts));
+    }
     HIP_TRY(hipEventRecord(r1, stream));
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventSynchronize(r1));
@@ -1588,7 +1595,7 @@ template <class R> struct Engine : EngineBase {
     (void)hipEventDestroy(r0);
     (void)hipEventDestroy(r1);
     if (region_ms) *region_ms = ms;
-    if (stage_avg_ms) *stage_avg_ms = tot / pairs_all.size();
+    if (stage_avg_ms) *stage_avg_ms = launches ? tot / pairs_all.size() : ms / (6 * attempts);
     KMT_TRY(fetch_state());
     fill_status(s);
     if (shadow.error) return fail(KMT_ERR_NUMERIC, "error norm is not finite");
