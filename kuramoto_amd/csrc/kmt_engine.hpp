@@ -350,28 +350,35 @@ template <class R> struct Engine : EngineBase {
     return KMT_OK;
   }
 
-  // `rows` rows of `width` bytes to host memory.  Pinned memory is written
-  // directly.  A pitched copy into pageable memory took 0.5 ms for six rows of
-  // 20 KB and 2 ms for 190 of 40 KB; here whole stretches of the source go to
-  // a pinned half buffer while the other half is spread over the caller's rows.
+  // `rows` rows of `width` bytes to the caller's memory.  What the runtime
+  // knows (pinned, device or managed memory) is written by one copy.  A pitched
+  // copy into pageable memory took 0.5 ms for six rows of 20 KB and 2 ms for
+  // 190 of 40 KB; there whole stretches of the source go to a pinned half
+  // buffer while the other half is spread over the caller's rows.  Without
+  // pinned memory to be had, the pitched copy it is.
   int drain_rows(void *dst, const void *src, size_t pitch, size_t width, size_t rows) {
     hipPointerAttribute_t at{};
     const hipError_t known = hipPointerGetAttributes(&at, dst);
-    if (known == hipSuccess && at.type == hipMemoryTypeHost) {
-      HIP_TRY(hipMemcpy2DAsync(dst, width, src, pitch, width, rows, hipMemcpyDeviceToHost, stream));
-      return KMT_OK;
-    }
     if (known != hipSuccess) (void)hipGetLastError();  // an address the runtime does not know is no error here
+    const bool direct = known == hipSuccess && at.type != hipMemoryTypeUnregistered;
     const size_t total = (rows - 1) * pitch + width;
     const size_t half = std::min(kStageMax, std::max<size_t>((total + 1) / 2, 4096));
-    if (stage_half < half) {
+    if (!direct && stage_half < half) {
       if (stage_buf) HIP_TRY(hipHostFree(stage_buf));
       stage_buf = nullptr;
       stage_half = 0;
-      HIP_TRY(hipHostMalloc((void **)&stage_buf, 2 * half, hipHostMallocDefault));
-      stage_half = half;
       for (hipEvent_t &e : stage_ev)
         if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      if (hipHostMalloc((void **)&stage_buf, 2 * half, hipHostMallocDefault) == hipSuccess) {
+        stage_half = half;
+      } else {
+        stage_buf = nullptr;
+        (void)hipGetLastError();
+      }
+    }
+    if (direct || !stage_buf) {
+      HIP_TRY(hipMemcpy2DAsync(dst, width, src, pitch, width, rows, direct ? hipMemcpyDefault : hipMemcpyDeviceToHost, stream));
+      return KMT_OK;
     }
     const size_t chunks = (total + stage_half - 1) / stage_half;
     auto start = [&](size_t c) -> int {
