@@ -863,9 +863,12 @@ struct kmt_batch {
   // fetched; before the first run they exist here only), and what the host
   // changed in them since - drained counts, an instance's or a factor's new
   // values - is in the device's once flush() has written them back
-  // (inst_dirty).  r_host: the rings as of then (r_valid).
+  // (inst_dirty).  r_host: what the rings held then (r_valid), r_pitch values
+  // per instance.
   bool inst_fresh = true, inst_dirty = false, r_valid = false;
-  float *r_host = nullptr;  // pinned, B x ring_cap
+  static constexpr size_t kRingStage = (size_t)1 << 20;
+  float *r_host = nullptr;  // pinned, kRingStage bytes
+  size_t r_pitch = 0;
   void *A = nullptr;
   size_t A_bytes = 0;
   std::vector<size_t> a_off;
@@ -1347,8 +1350,6 @@ struct kmt_batch {
       vhalf = B;
     }
     inst_fresh = inst_dirty = r_valid = false;
-    if (r_host) HIP_TRY(hipHostFree(r_host));
-    r_host = nullptr;
     HIP_TRY(hipMemcpyAsync(inst, host_inst.data(), sizeof(BInst) * B, hipMemcpyHostToDevice, stream));
     // k1 = f(y) for every instance, then the first stage-2 vectors
     dim3 g2((unsigned)nblk, (unsigned)B);
@@ -1456,17 +1457,32 @@ struct kmt_batch {
     const int ready = host_inst[b].ring_count;
     const int n = std::min(std::max(max_n, 0), ready);
     if (ready > 0) {
-      // the rings of all instances in one copy: drains of the others follow
+      // what the rings of all instances hold in one copy (drains of the others
+      // follow), while that is little; else this one's alone
       if (!r_valid) {
-        if (!r_host) HIP_TRY(hipHostMalloc((void **)&r_host, sizeof(float) * (size_t)B * ring_cap, hipHostMallocDefault));
         int most = 0;
         for (const BInst &in : host_inst) most = std::max(most, in.ring_count);
-        HIP_TRY(hipMemcpy2DAsync(r_host, sizeof(float) * ring_cap, r_ring, sizeof(float) * ring_cap, sizeof(float) * most, B,
-                                 hipMemcpyDeviceToHost, stream));
-        HIP_TRY(hipStreamSynchronize(stream));
-        r_valid = true;
+        if (sizeof(float) * (size_t)B * most <= kRingStage && !r_host &&
+            hipHostMalloc((void **)&r_host, kRingStage, hipHostMallocDefault) != hipSuccess) {
+          r_host = nullptr;
+          (void)hipGetLastError();
+        }
+        if (sizeof(float) * (size_t)B * most <= kRingStage && r_host) {
+          r_pitch = most;
+          HIP_TRY(hipMemcpy2DAsync(r_host, sizeof(float) * r_pitch, r_ring, sizeof(float) * ring_cap, sizeof(float) * most, B,
+                                   hipMemcpyDeviceToHost, stream));
+          HIP_TRY(hipStreamSynchronize(stream));
+          r_valid = true;
+        }
       }
-      float *mine = r_host + (size_t)b * ring_cap;
+      std::vector<float> alone;
+      float *mine = r_valid ? r_host + (size_t)b * r_pitch : nullptr;
+      if (!r_valid) {
+        alone.resize(ready);
+        mine = alone.data();
+        HIP_TRY(hipMemcpyAsync(mine, r_ring + (size_t)b * ring_cap, sizeof(float) * ready, hipMemcpyDeviceToHost, stream));
+        HIP_TRY(hipStreamSynchronize(stream));
+      }
       for (int q = 0; q < n; ++q) r[q] = mine[q];
       if (n > 0) {
         if (n < ready) {  // keep the unread values at the front
