@@ -74,6 +74,8 @@ int kmt_fail(int code, const char *fmt, ...) {
   vsnprintf(buf, sizeof(buf), fmt, ap);
   va_end(ap);
   g_last_error = buf;
+  // reported here: not once more by the next call that asks the runtime
+  if (code == KMT_ERR_HIP || code == KMT_ERR_MEMORY) (void)hipGetLastError();
   return code;
 }
 

@@ -1316,6 +1316,11 @@ struct kmt_batch {
     if (rcap < 1) return kmt_fail(KMT_ERR_ARG, "ring_rows must be >= 1");
     HIP_TRY(hipStreamSynchronize(stream));
     drop_graphs();
+    KMT_TRY(fetch());
+    begun = 0;  // no run if the rest fails: its buffers are replaced one by one
+    for (BInst &in : host_inst) in.ring_count = 0;
+    inst_dirty = true;
+    r_valid = false;
     KMT_TRY(ensure_P());
     KMT_TRY(build_items());
     if (shared && !tiled) default_split();

@@ -599,12 +599,29 @@ template <class R> struct Engine : EngineBase {
     if (k_ < 0) return fail(KMT_ERR_ARG, "rank K must be >= 0");
     HIP_TRY(hipStreamSynchronize(stream));  // the buffers below may be in use by queued work
     drop_graphs();
+    drop_factor();
+    const int rc = make_factor(Xv, wv, k_);
+    if (rc != KMT_OK) {  // all of it or none: coupling_ready asks for X alone
+      drop_factor();
+      return rc;
+    }
+    if (factored == KMT_LOWRANK_REBUILD) {  // keep the mode, if the new rank allows it
+      factored = KMT_LOWRANK_CONTRACT;
+      return use_factored(KMT_LOWRANK_REBUILD);
+    }
+    return KMT_OK;
+  }
+
+  void drop_factor() {
     if (X) { (void)hipFree(X); X = nullptr; }
     if (w) { (void)hipFree(w); w = nullptr; }
     if (XT) { (void)hipFree(XT); XT = nullptr; }
     if (lr_part) { (void)hipFree(lr_part); lr_part = nullptr; }
     if (lr_G) { (void)hipFree(lr_G); lr_G = nullptr; }
     drop_sign();
+  }
+
+  int make_factor(const void *Xv, const void *wv, int k_) {
     K = k_;
     const long kk = std::max(K, 1);
     X_host.assign((const R *)Xv, (const R *)Xv + (size_t)N * K);
@@ -628,10 +645,6 @@ template <class R> struct Engine : EngineBase {
     HIP_TRY(hipMalloc((void **)&lr_G, sizeof(double) * 2 * kk));
     HIP_TRY(hipMemsetAsync(lr_G, 0, sizeof(double) * 2 * kk, stream));
     HIP_TRY(hipStreamSynchronize(stream));
-    if (factored == KMT_LOWRANK_REBUILD) {  // keep the mode, if the new rank allows it
-      factored = KMT_LOWRANK_CONTRACT;
-      return use_factored(KMT_LOWRANK_REBUILD);
-    }
     return KMT_OK;
   }
 
@@ -689,12 +702,7 @@ template <class R> struct Engine : EngineBase {
       return fail(KMT_ERR_ARG, "the packed sign factor needs N, K <= %ld (N=%ld, K=%d)", kSignMaxDim, N, k_);
     HIP_TRY(hipStreamSynchronize(stream));
     drop_graphs();
-    if (X) { (void)hipFree(X); X = nullptr; }
-    if (w) { (void)hipFree(w); w = nullptr; }
-    if (XT) { (void)hipFree(XT); XT = nullptr; }
-    if (lr_part) { (void)hipFree(lr_part); lr_part = nullptr; }
-    if (lr_G) { (void)hipFree(lr_G); lr_G = nullptr; }
-    drop_sign();
+    drop_factor();
     if (factored == KMT_LOWRANK_REBUILD) factored = KMT_LOWRANK_CONTRACT;
     K = k_;
     X_host.clear();
@@ -889,6 +897,12 @@ template <class R> struct Engine : EngineBase {
   }
 
   int coupling_ready() const { return factored ? (X != nullptr || sign) : (A != nullptr); }
+  // before attempts are launched: kmt_use_factored and failed uploads can take
+  // the coupling away from a run between advances
+  int still_coupled() const {
+    if (!coupling_ready()) return fail(KMT_ERR_STATE, "no adjacency: call kmt_set_adjacency, kmt_build_adjacency or kmt_set_factor + kmt_use_factored");
+    return KMT_OK;
+  }
 
   // workgroups of one resident round of the balanced variant (<= N rows)
   template <class S, int ROWS, bool NT> int balanced_grid() {
@@ -1256,6 +1270,7 @@ template <class R> struct Engine : EngineBase {
   }
   // n attempts of the run
   int launch_attempts(int n) {
+    KMT_TRY(still_coupled());
     ensure_variant();
     if (small_path()) {
       SmallArgs<R> a;
@@ -1363,6 +1378,7 @@ template <class R> struct Engine : EngineBase {
     if (rcap < 1) return fail(KMT_ERR_ARG, "ring_rows must be >= 1");
     HIP_TRY(hipStreamSynchronize(stream));
     drop_graphs();
+    begun = 0;  // no run if the rest fails: its buffers are replaced one by one
     if (t_eval) { (void)hipFree(t_eval); t_eval = nullptr; }
     if (ring) { (void)hipFree(ring); ring = nullptr; }
     if (r_ring) { (void)hipFree(r_ring); r_ring = nullptr; }
@@ -1566,6 +1582,7 @@ template <class R> struct Engine : EngineBase {
     KMT_TRY(fetch_state());
     if (attempts > shadow.times_cap - shadow.times_count)
       return fail(KMT_ERR_ARG, "attempts exceed the accepted-step log capacity; drain kmt_read_times first");
+    KMT_TRY(still_coupled());
     ensure_variant();
     const bool launches = !small_path();  // the one-workgroup form has no stage launches to time
     std::vector<std::pair<hipEvent_t, hipEvent_t>> pairs_all(launches ? 6 * attempts : 0);
