@@ -273,7 +273,8 @@ __global__ __launch_bounds__(WAVES * kWave) void bgemm_kernel(const T *At, long 
       }
       __builtin_amdgcn_sched_group_barrier(0x008, F, 0);
     } else {
-      // Two or more bands: a set is the MT fragments of one (k-step, hi or
+      // Two or more bands (the shapes of 512 rows, which the tuner or the
+      // caller picks; the default has one): a set is the MT fragments of one (k-step, hi or
       // lo); set s + 1 is read from LDS while the MT NT MFMAs of set s run.
       // Reading each fragment right before its MFMAs left the LDS latency
       // exposed once per set: 512-row workgroups, B = 64, N = 20000, split 6:

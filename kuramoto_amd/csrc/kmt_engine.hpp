@@ -267,8 +267,9 @@ template <class R> struct Engine : EngineBase {
   }
 
   // Rows per error partial.  16-bit entries: 16; the working precision: 8 (the
-  // grouping of the FP64 register-rebuild kernel, whose runs are the dense
-  // ones' bit for bit); 4 for matrices of 4096 rows up to 128 MB.
+  // grouping of the FP64 register-rebuild kernel for K <= 8, whose runs are
+  // the dense ones' bit for bit); 4 from N = 4096 on up to 128 MB.  Any fixed
+  // choice would do; another one is another sequence of steps.
   int error_rows() const {
     if (pinned) return tune_rows;
     if (N >= 4096 && (double)N * (double)N * (double)elem_bytes(storage) <= 128e6) return 4;

@@ -82,8 +82,9 @@ struct AdamArgs {
 //   waves 64..71  dW1[l][j] = sum_s D1[s][l] X[s][j]      V = D1, U = X column j
 //   waves 72..75  db1[l], db2[l] (V = D1, D2), dW3[l] (V = H2, U = D3), db3 (U = D3)
 // The sum runs over s in order, one fma per sample, so that training gives
-// the same bits whatever the shape of the launch; that chain (4 to 8 cycles
-// per sample) is the bound.  What it needs is its operands on time: one
+// the same bits whatever the shape of the launch; the chain itself would take
+// 4 to 8 cycles per sample.  What bounds it are its operands, about 30 cycles
+// per sample: a wave waits for a cache round trip per register set.  One
 // thread per parameter with both loads inside the loop waited for memory
 // once per few samples (227 us for 1024 samples).  Here V is loaded kMlpU
 // samples at a time into one of two register sets while the other is summed
